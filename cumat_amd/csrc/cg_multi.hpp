@@ -475,6 +475,12 @@ __device__ __forceinline__ void cg_k1_snapshot(CgState<T>* st, int bb)
     }
 }
 
+}  // namespace cm
+
+#include "cg_dia.hpp"  // K1 over the diagonals; uses the state and the snapshot above
+
+namespace cm {
+
 // ---------------------------------------------------------------- K1 (three-launch form)
 // tmp = A p, per-block partial p.tmp
 template <typename VT, typename T, int MNT = 0>
@@ -1078,9 +1084,12 @@ template <typename VT, typename T>
 static void launch_cg_iteration(cm_ctx_t ctx, int n, int B, int G1, int G2, const int* JA, const int* IA,
                                 const VT* vals, long long vstride, const T* invd, int istride, T* p, T* t, T* x, T* r,
                                 T* part1, T* part2, CgState<T>* st, const T* diag, const DenseOp<T>* dense,
-                                const T* r0, CgMirror* mirror, int x0_zero, const BlockOp* block = nullptr)
+                                const T* r0, CgMirror* mirror, int x0_zero, const BlockOp* block = nullptr,
+                                const DiaArgs* da = nullptr, const VT* dia = nullptr)
 {
-    if (block) {
+    if (da) {
+        launch_cg_dia<VT, T>(ctx->stream, n, B, G1, *da, dia, p, t, part1, st, diag);
+    } else if (block) {
         if constexpr (std::is_same<T, float>::value) launch_cg_bcsr(ctx->stream, *block, B, G1, p, t, part1, st);
     } else if (dense && dense->row_major)
         cg_dense_kernel<T, true><<<dim3(G1, B), CG_BS, 0, ctx->stream>>>(n, dense->A, dense->bstride, p, t, part1, st);
@@ -1124,6 +1133,28 @@ struct CgBatchOpts {
     const BlockOp* block = nullptr;  // a block-CSR operator replaces the CSR matrix (FP32)
 };
 
+// Queues the layout by diagonals; *dia stays NULL where it does not pay or
+// no memory is left (the solve then keeps the CSR product).
+template <typename VT>
+static int cg_dia_prepare(cm_ctx_t ctx, Temps& tmp, int n, int nnz, int nb, const int* JA, const int* IA,
+                          const VT* vals, long long vstride, long long ld, void* pinned_dev, VT** dia)
+{
+    const long long cap = (long long)nnz + nnz / 4 + 8 * 32;
+    void* buf = nullptr;
+    const size_t plan_bytes = 256;
+    static_assert(sizeof(DiaPlan) <= 256, "plan block");
+    if (tmp.get(plan_bytes + sizeof(VT) * (size_t)cap * nb, &buf) != CM_OK) return CM_OK;
+    DiaPlan* plan = (DiaPlan*)buf;
+    DiaPlan* host = (DiaPlan*)((char*)pinned_dev + CM_PINNED_BYTES / 2);
+    *dia = (VT*)((char*)buf + plan_bytes);
+    cg_dia_detect_kernel<<<1, CG_DIA_DETECT_BS, 0, ctx->stream>>>(n, JA, IA, ld, cap, plan, host);
+    CM_LAUNCH_CHECK();
+    cg_dia_convert_kernel<VT><<<dim3(div_up(ld, CG_DIA_BS), nb), CG_DIA_BS, 0, ctx->stream>>>(
+        n, JA, IA, vals, vstride, ld, *dia, plan, host);
+    CM_LAUNCH_CHECK();
+    return CM_OK;
+}
+
 template <typename VT, typename T>
 static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, const int* IA, const VT* vals,
                            const T* invd, const T* b, T* x, int use_guess, double tol, int max_iter, int* iters_out,
@@ -1147,7 +1178,7 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     // 512-row blocks with the same grid.
     const int gcap = std::max(8, CG_GMAX / B);
     // (a block operator walks 64-block-row chunks of its rows)
-    const int G1 = walk_grid(div_up(div_up(block ? block->rows : n, 64), CG_BS / 64), gcap);
+    int G1 = walk_grid(div_up(div_up(block ? block->rows : n, 64), CG_BS / 64), gcap);
     const int G2 = walk_grid(div_up(n, (long long)CG_BS * CG_VPT), std::min(gcap, CG_G2MAX));
     // reduce_pairs_batched folds at most CG_PPT + 1 pairs per thread
     CM_REQUIRE(B == 1 || G2 <= (CG_PPT + 1) * (CG_BS / B), CM_E_UNSUPPORTED, "CG: grid %d too large for %d batches",
@@ -1202,8 +1233,10 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     void* mirror_host = nullptr;
     void* mirror_dev = nullptr;
     CM_TRY(pinned(ctx, &mirror_host, &mirror_dev));
-    static_assert(sizeof(CgMirror) <= CM_PINNED_BYTES, "the solve mirror must fit the pinned page");
+    static_assert(sizeof(CgMirror) <= CM_PINNED_BYTES / 2 && sizeof(DiaPlan) <= CM_PINNED_BYTES / 2,
+                  "mirror and plan share the pinned page");
     volatile CgMirror* hm = (volatile CgMirror*)mirror_host;
+    volatile DiaPlan* hplan = (volatile DiaPlan*)((char*)mirror_host + CM_PINNED_BYTES / 2);
     CgMirror* mirror = (CgMirror*)mirror_dev;
     // the previous solve on this context left its final state here
     hm->status = CG_RUNNING;
@@ -1265,12 +1298,30 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
         }
     };
     int it = 0;
+    // K1 over the diagonals (cg_dia.hpp): laid out after the first chunk if
+    // enough iterations are left to pay for it, used from CG_DIA_FROM on
+    const bool try_dia = !fused && !dense && !block && max_iter >= CG_DIA_FROM + 2 * CG_CHUNK && nnz > 0;
+    const long long dia_ld = ((long long)n + 7) / 8 * 8;
+    DiaArgs da{};
+    VT* dia = nullptr;
+    const DiaArgs* dia_on = nullptr;
     while (it < max_iter) {
         int todo = std::min(CG_CHUNK, max_iter - it);
+        if (try_dia && it == CG_CHUNK)
+            CM_TRY((cg_dia_prepare<VT>(ctx, tmp, n, nnz, nbi, JA, IA, vals, vstride, dia_ld, mirror_dev, &dia)));
+        if (dia && !dia_on && it == CG_DIA_FROM && hplan->count > 0 && !hplan->bad) {
+            // the host has waited for an iteration queued behind the conversion
+            da.count = hplan->count;
+            da.ld = dia_ld;
+            da.bstride = vstride ? da.count * dia_ld : 0;
+            for (int d = 0; d < da.count; ++d) da.off[d] = hplan->off[d];
+            dia_on = &da;
+            G1 = walk_grid(div_up(n, cg_dia_rows_per_block(n)), gcap);
+        }
         for (int k = 0; k < todo; ++k, ++it) {
             if (!fused) {
                 launch_cg_iteration<VT, T>(ctx, n, B, G1, G2, JA, IA, vals, vstride, invd, istride, p, t, x, r, part1,
-                                           part2, st, diag, dense, r0, mirror, x0_zero, block);
+                                           part2, st, diag, dense, r0, mirror, x0_zero, block, dia_on, dia);
                 continue;
             }
             T* pcur = pbuf[it & 1];
