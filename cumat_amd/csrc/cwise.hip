@@ -15,8 +15,7 @@
 // Also here: the pre-instantiated linear combination (k <= 16 streams) and
 // evaluation into the non-zeros of a CSR matrix
 // (CwiseCSREvaluationKernel, cuMat/src/SparseEvaluation.h:14-34).
-#include "cwise_core.hpp"
-#include "jit.hpp"
+#include "cwise_tile.hpp"
 
 #include <cinttypes>
 
@@ -276,7 +275,6 @@ static int launch_csr_w(cm_ctx_t ctx, const CwProgram& P, const int* JA, const i
 // non-temporal loads and stores where the interpreter takes them, the
 // same per-element semantics (cwise_ops.hpp). Returns CM_OK when launched,
 // JIT_DECLINED when the interpreter should run the program.
-constexpr int JIT_DECLINED = 1;
 
 struct JitCwiseArgs {
     const void* leaf[CM_CWISE_MAX_LEAVES];
@@ -812,6 +810,8 @@ static int cwise_dense(cm_ctx_t ctx, const cm_leaf* leaves, int nleaves, const c
     }
     // (also programs with strided or broadcast leaves, coordinates compiled in)
     if (P.dst_direct && cm::jit::want(n)) {
+        const int t = flat ? cm::JIT_DECLINED : cm::jit_cwise_tile(ctx, P, wide);
+        if (t != cm::JIT_DECLINED) return t;
         const int s = cm::jit_cwise_flat(ctx, P, 0, nullptr, wide);
         if (s != cm::JIT_DECLINED) return s;
     }
