@@ -17,14 +17,11 @@
 // programs) elements per thread and pass, folds them in a fixed order, and
 // long segments fold their per-chunk partials in a second launch, the same
 // order every run (results are bit-reproducible).
-#include "cwise_core.hpp"
-#include "jit.hpp"
+#include "rxcol.hpp"
 
 #include <limits>
 
 namespace cm {
-
-constexpr int RX_BS = 256;
 
 template <typename Op, typename T> struct RxIdentity;
 template <typename T> struct RxIdentity<OpSum, T> { __device__ static T v() { return T(0); } };
@@ -35,16 +32,6 @@ template <typename T> struct RxIdentity<OpAll, T> { __device__ static T v() { re
 template <typename T> struct RxIdentity<OpAny, T> { __device__ static T v() { return T(0); } };
 template <typename T> struct RxIdentity<OpBand, T> { __device__ static T v() { return ~T(0); } };
 template <typename T> struct RxIdentity<OpBor, T> { __device__ static T v() { return T(0); } };
-
-// Virtual order: up to three kept axes (kdim / kaxis, innermost first, in
-// the output layout's order) and up to three reduced axes (rdim / raxis).
-// Axis ids: 0 row, 1 column, 2 batch.
-struct RxShape {
-    long long kdim[3], rdim[3];
-    int kaxis[3], raxis[3];
-    int nk, nr;
-    long long L, nseg;
-};
 
 template <typename T> __device__ __forceinline__ T rx_get(const Reg<false>& r, int k);
 template <> __device__ __forceinline__ float rx_get<float>(const Reg<false>& r, int k) { return getf(r, k); }
@@ -209,17 +196,6 @@ static bool rx_any_virtual(const CwProgram& P, const RxShape& SH)
     }
     return false;
 }
-
-constexpr int RX_JIT_DECLINED = 1;
-
-// Arguments of the generated reduction kernel cm_jit_reduce.
-struct JitRxArgs {
-    const void* leaf[CM_CWISE_MAX_LEAVES];
-    void* partials;
-    void* out;
-    long long L, chunk;
-    int nchunk, pad;
-};
 
 template <typename Op> struct RxOpName;
 template <> struct RxOpName<OpSum> { static const char* get() { return "cm::OpSum"; } };
@@ -503,6 +479,29 @@ int jit_reduce_strided_source(const CwProgram& P, const RxShape& SH, std::string
     return CM_OK;
 }
 
+// The identity where T may also be double.
+template <typename Op, typename T>
+static std::string rx_identity_wide_src()
+{
+    if (!std::is_same<T, double>::value) return rx_identity_src<Op, T>();
+    if (std::is_same<Op, OpMin>::value) return "__longlong_as_double(0x7fefffffffffffffll)";
+    if (std::is_same<Op, OpMax>::value) return "__longlong_as_double((long long)0xffefffffffffffffull)";
+    if (std::is_same<Op, OpProd>::value || std::is_same<Op, OpAll>::value) return "1.0";
+    return "0.0";
+}
+
+// How the reduction of Op in T, stored as S, is spelled (rxcol.hip).
+template <typename Op, typename T, typename S>
+static RxNames rx_names()
+{
+    auto name = [](bool f, bool i, bool d) { return f ? "float" : (i ? "int" : (d ? "double" : "unsigned char")); };
+    return {RxOpName<Op>::get(),
+            name(std::is_same<T, float>::value, std::is_same<T, int>::value, std::is_same<T, double>::value),
+            name(std::is_same<S, float>::value, std::is_same<S, int>::value, std::is_same<S, double>::value),
+            std::is_same<T, float>::value ? "getf" : (std::is_same<T, int>::value ? "geti" : "getd"),
+            rx_identity_wide_src<Op, T>()};
+}
+
 // Source and key of the generated reduction of a 64-bit program (FP64
 // leaves or instructions): the kernel of reduce_expr_kernel<Op, T, S, true,
 // NL, FLAT> -- 4 consecutive elements of the virtual order per thread and
@@ -598,15 +597,7 @@ int jit_reduce_wide_source(const CwProgram& P, const RxShape& SH, std::string& k
     std::string prog;
     if (!jit::program_body(P, namep, prog)) return RX_JIT_DECLINED;
     const char* get = std::is_same<T, float>::value ? "getf" : (std::is_same<T, int>::value ? "geti" : "getd");
-    std::string ident;
-    if (std::is_same<T, double>::value) {
-        if (std::is_same<Op, OpMin>::value) ident = "__longlong_as_double(0x7fefffffffffffffll)";
-        else if (std::is_same<Op, OpMax>::value) ident = "__longlong_as_double((long long)0xffefffffffffffffull)";
-        else if (std::is_same<Op, OpProd>::value || std::is_same<Op, OpAll>::value) ident = "1.0";
-        else ident = "0.0";
-    } else {
-        ident = rx_identity_src<Op, T>();
-    }
+    const std::string ident = rx_identity_wide_src<Op, T>();
     body = std::string("typedef ") + tname + " TT;\ntypedef " + sname + " SS;\ntypedef " + RxOpName<Op>::get() +
            " OP;\n"
            "struct JitRxArgs { const void* leaf[" + std::to_string(CM_CWISE_MAX_LEAVES) +
@@ -682,6 +673,11 @@ static int launch_reduce_expr(cm_ctx_t ctx, const CwProgram& P0, const RxShape& 
     bool done = false;
     {
         if (jit::want(SH.L * SH.nseg)) {
+            const int st = rx_column_launch(ctx, P, SH, rx_names<Op, T, S>(), W, spread && !W, nchunk, chunk, part, out);
+            if (st != CM_OK && st != RX_JIT_DECLINED) return st;
+            done = st == CM_OK;
+        }
+        if (!done && jit::want(SH.L * SH.nseg)) {
             // everything the generators read (the front cache's signature)
             std::string sig(W ? "rxw" : "rx");
             sig += RxOpName<Op>::get();
