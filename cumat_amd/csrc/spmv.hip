@@ -10,10 +10,15 @@
 #include "spmv_core.hpp"
 #include "spmv_wave.hpp"
 
+#include <algorithm>
+
 namespace cm {
 
 constexpr int SPMV_BS = 256;
 constexpr int SPMV_EPT = 8;   // staged non-zeros per lane (8 per row on average)
+// Vectors are multiplied together from this many (wavefronts x vectors) on:
+// below, 8 vectors of 300^2 (11 k) take 7.5 us either way.
+constexpr long long SPMV_MULTI_WAVES = 16384;
 
 template <typename VT, typename T>
 __global__ __launch_bounds__(SPMV_BS) void csr_spmv_kernel(int rows, int cols, int nnz,
@@ -48,6 +53,107 @@ __global__ __launch_bounds__(SPMV_BS) void csr_spmv_kernel(int rows, int cols, i
         if (!more) break;
         cur = nxt;
         w.next();
+    }
+}
+
+// The product of NB vectors that share the matrix values (blockIdx.y counts
+// groups of NB; the last group may hold fewer): the chunk's indices and values
+// are read once and stay in registers while one vector after the other is
+// gathered and summed. Same sums as csr_spmv_kernel. Measured on MI355X, us, a
+// launch of one vector each / together: 1024^2 FP32 2 vectors 24.2 / 19.9, 4
+// 45.1 / 29.2, 8 84.6 / 50.8; 100^3 FP64 7 points 3 vectors 64.3 / 39.9. One
+// vector stays with csr_spmv_kernel: the same code here takes 68 registers
+// instead of 62, one wavefront less per SIMD, and 62 us instead of 44 at 2048^2.
+template <typename VT, typename T, int NB>
+__global__ __launch_bounds__(SPMV_BS, sizeof(T) == 4 ? 8 : 4) void csr_spmv_multi_kernel(int rows, int cols, int batches,
+                                                           const int* __restrict__ JA,
+                                                           const int* __restrict__ IA,
+                                                           const VT* __restrict__ vals,
+                                                           const T* __restrict__ x, T* __restrict__ y, int mode)
+{
+    constexpr int WPB = SPMV_BS / 64;
+    __shared__ T lds[WPB][SPMV_EPT * 64];
+    T* slice = lds[threadIdx.x >> 6];
+    const int lane = threadIdx.x & 63;
+    const int b0 = blockIdx.y * NB;
+    const int nb = min(NB, batches - b0);  // a vector past the last one repeats the group's first
+    const VT* v = vals;
+    const T* xb = x + (long long)b0 * cols;
+    T* yb = y + (long long)b0 * rows;
+    ChunkWalk w(div_up_dev(rows, 64), WPB);
+    if (!w.valid()) return;  // wave-uniform; no block barrier below
+    WaveChunk<VT, SPMV_EPT> cur, nxt;
+    chunk_load(cur, JA, IA, v, w.cur * 64, rows);
+    for (;;) {
+        const int nc = w.peek_next();
+        const bool more = nc < w.hi;
+        if (more) chunk_load(nxt, JA, IA, v, nc * 64, rows);  // in flight during the gathers below
+        T acc[NB];
+        chunk_compute_multi<VT, T, SPMV_EPT, NB>(
+            cur, JA, IA, v, [=](int b, int c) { return xb[(b < nb ? (long long)b * cols : 0) + c]; }, slice, acc);
+        if (lane < cur.nr) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if (b >= nb) break;
+                T* yy = yb + (long long)b * rows + cur.r0 + lane;
+                if (mode == CM_ASSIGN) __builtin_nontemporal_store(acc[b], yy);
+                else *yy = assign_mode<T>(mode, *yy, acc[b]);
+            }
+        }
+        if (!more) break;
+        cur = nxt;
+        w.next();
+    }
+}
+
+// Rows of more than SPMV_EPT entries on average: every chunk of 64 rows is
+// taken in windows of SPMV_EPT * 64 entries. Chunks with a row of more than
+// SPMV_ROW_MAX entries go row by row: one lane would add such a row while the
+// others wait.
+//
+// Row by row, a row of 27 entries is one load per lane, 37 lanes idle, and a
+// wave reduction; the next row's loads wait for it. Measured on MI355X, us, row
+// by row / windows: 27 points, 572 k rows, FP64 136 / 45.5 (one vector), 332 /
+// 71.8 (three, the windows read once for all), FP32 107 / 34.1; 200 k rows of 1
+// to 39 entries FP32 41.5 / 19.3. Without the next window's loads in flight
+// 54.8, 78.8, 46.5 and 23.8.
+constexpr int SPMV_ROW_MAX = 128;
+template <typename VT, typename T, int NB>
+__global__ __launch_bounds__(SPMV_BS) void csr_spmv_wide_kernel(int rows, int cols, int nnz, int batches,
+                                                                const int* __restrict__ JA,
+                                                                const int* __restrict__ IA,
+                                                                const VT* __restrict__ vals, int vals_batched,
+                                                                const T* __restrict__ x, int x_batched,
+                                                                T* __restrict__ y, int mode)
+{
+    constexpr int WPB = SPMV_BS / 64;
+    __shared__ T lds[WPB][SPMV_EPT * 64];
+    T* slice = lds[threadIdx.x >> 6];
+    const int lane = threadIdx.x & 63;
+    const int b0 = blockIdx.y * NB;
+    const int nb = min(NB, batches - b0);
+    const VT* v = vals + (vals_batched ? (long long)b0 * nnz : 0);
+    const T* xb = x + (x_batched ? (long long)b0 * cols : 0);
+    T* yb = y + (long long)b0 * rows;
+    auto xg = [=](int b, int c) { return xb[(b < nb ? (long long)b * cols : 0) + c]; };
+    for (ChunkWalk w(div_up_dev(rows, 64), WPB); w.valid(); w.next()) {
+        const int r0 = w.cur * 64, nr = min(64, rows - r0);
+        const int s = JA[r0], e = JA[r0 + nr];
+        const int rb = lane < nr ? JA[r0 + lane] : 0, re = lane < nr ? JA[r0 + lane + 1] : 0;
+        T acc[NB];
+        if (wave_reduce<OpMax>(re - rb) <= SPMV_ROW_MAX)
+            chunk_windows<VT, T, SPMV_EPT, NB>(s, e, rb, re, IA, v, xg, slice, acc);
+        else
+            chunk_rows<VT, T, NB>(r0, nr, JA, IA, v, xg, acc);
+        if (lane < nr) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if (b >= nb) break;
+                T* yy = yb + (long long)b * rows + r0 + lane;
+                if (mode == CM_ASSIGN) __builtin_nontemporal_store(acc[b], yy);
+                else *yy = assign_mode<T>(mode, *yy, acc[b]);
+            }
+        }
     }
 }
 
@@ -147,9 +253,31 @@ static int launch_csr(cm_ctx_t ctx, int rows, int cols, int nnz, int batches, co
         const char* s = getenv("CUMAT_SPMV_GRID");
         return (s && atoi(s) >= 8) ? atoi(s) : 2048;
     }();
-    dim3 grid(walk_grid(div_up(div_up(rows, 64), SPMV_BS / 64), gmax), batches);
-    csr_spmv_kernel<VT, T><<<grid, SPMV_BS, 0, ctx->stream>>>(rows, cols, nnz, JA, IA, (const VT*)vals, vb,
-                                                              (const T*)x, xb, (T*)y, mode);
+    const int g = walk_grid(div_up(div_up(rows, 64), SPMV_BS / 64), gmax);
+    // more entries than a chunk holds: the windows
+    const bool wide = nnz > (long long)SPMV_EPT * rows;
+#define CM_WIDE(NB)                                                                                             \
+    csr_spmv_wide_kernel<VT, T, NB><<<dim3(g, (batches + NB - 1) / NB), SPMV_BS, 0, ctx->stream>>>(             \
+        rows, cols, nnz, batches, JA, IA, (const VT*)vals, vb, (const T*)x, xb, (T*)y, mode)
+#define CM_MULTI(NB)                                                                                            \
+    csr_spmv_multi_kernel<VT, T, NB><<<dim3(g, (batches + NB - 1) / NB), SPMV_BS, 0, ctx->stream>>>(            \
+        rows, cols, batches, JA, IA, (const VT*)vals, (const T*)x, (T*)y, mode)
+    // vectors that share the values are multiplied together, as long as the
+    // groups still fill the chip (a wavefront takes 64 rows)
+    const long long waves = (long long)div_up(rows, 64) * batches;
+    const int nb = (vb || !xb || waves < SPMV_MULTI_WAVES) ? 1 : std::min(batches, 4);
+    if (nb == 1 && wide) CM_WIDE(1);
+    else if (nb == 1)
+        csr_spmv_kernel<VT, T><<<dim3(g, batches), SPMV_BS, 0, ctx->stream>>>(
+            rows, cols, nnz, JA, IA, (const VT*)vals, vb, (const T*)x, xb, (T*)y, mode);
+    else if (nb == 2 && wide) CM_WIDE(2);
+    else if (nb == 2) CM_MULTI(2);
+    else if (nb == 3 && wide) CM_WIDE(3);
+    else if (nb == 3) CM_MULTI(3);
+    else if (wide) CM_WIDE(4);
+    else CM_MULTI(4);
+#undef CM_WIDE
+#undef CM_MULTI
     CM_LAUNCH_CHECK();
     return CM_OK;
 }

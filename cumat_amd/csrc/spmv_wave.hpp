@@ -13,7 +13,8 @@
 // index/value loads of one chunk overlap the gathers of the previous one and
 // every wavefront keeps two chunks of loads in flight.
 // Chunks with more non-zeros fall back to one row at a time per wavefront
-// (lanes stride the row, fixed-order DPP reduction).
+// (chunk_rows); a matrix with many of them has a kernel of its own
+// (chunk_windows).
 // Chunks are assigned so that each XCD owns a contiguous range of rows:
 // stencil neighbours of a chunk are then resident in the same L2.
 #pragma once
@@ -81,6 +82,120 @@ __device__ __forceinline__ void chunk_load(WaveChunk<VT, EPT>& C, const int* __r
             C.col[j] = ok ? ld_matrix<(NT & 1) != 0>(IA + k) : 0;
             C.v[j] = ok ? ld_matrix<(NT & 2) != 0>(vals + k) : VT(0);
         }
+    }
+}
+
+// (A x)[r0 + lane] of a chunk one row at a time (lanes stride the row,
+// fixed-order DPP reduction), for the NB vectors xg(b, col).
+template <typename VT, typename T, int NB, typename XG>
+__device__ __forceinline__ void chunk_rows(int r0, int nr, const int* __restrict__ JA, const int* __restrict__ IA,
+                                           const VT* __restrict__ vals, XG xg, T (&out)[NB])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        out[b] = T(0);
+        for (int i = 0; i < nr; ++i) {
+            const int a = JA[r0 + i], e = JA[r0 + i + 1];
+            T s = T(0);
+            for (int k = a + lane; k < e; k += 64) s += Load<VT, T>::get(vals, k) * xg(b, IA[k]);
+            s = wave_reduce<OpSum>(s);
+            if (lane == i) out[b] = s;
+        }
+    }
+}
+
+// The same through windows of EPT * 64 entries: a window's entries are loaded
+// and multiplied like a narrow chunk's, and a lane adds the part of its row
+// that lies in the window in four chains. Row lane: entries [rb, re).
+template <typename VT, typename T, int EPT, int NB, typename XG>
+__device__ __forceinline__ void chunk_windows(int s, int end, int rb, int re, const int* __restrict__ IA,
+                                              const VT* __restrict__ vals, XG xg, T* slice, T (&out)[NB])
+{
+    constexpr int WIN = EPT * 64;
+    const int lane = threadIdx.x & 63;
+    T part[NB][4];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) part[b][q] = T(0);
+    int ncol[EPT];
+    VT nv[EPT];
+    auto load = [&](int w0) {
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) {
+            const int k = w0 + lane + 64 * j;
+            const bool ok = k < end;
+            ncol[j] = ok ? __builtin_nontemporal_load(IA + k) : 0;
+            nv[j] = ok ? __builtin_nontemporal_load(vals + k) : VT(0);
+        }
+    };
+    load(s);
+    for (int w0 = s; w0 < end; w0 += WIN) {
+        int col[EPT];
+        VT v[EPT];
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) {
+            col[j] = ncol[j];
+            v[j] = nv[j];
+        }
+        if (w0 + WIN < end) load(w0 + WIN);  // in flight during this window's gathers
+        const int a = max(rb, w0) - w0, e = min(re, w0 + WIN) - w0;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            T xv[EPT];
+#pragma unroll
+            for (int j = 0; j < EPT; ++j) xv[j] = (w0 + lane + 64 * j < end) ? xg(b, col[j]) : T(0);
+#pragma unroll
+            for (int j = 0; j < EPT; ++j) slice[lane + 64 * j] = Load<VT, T>::get(v, j) * xv[j];
+            __builtin_amdgcn_wave_barrier();  // as in chunk_compute
+            int k = a;
+            for (; k + 3 < e; k += 4)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) part[b][q] += slice[k + q];
+            for (; k < e; ++k) part[b][0] += slice[k];
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) out[b] = (part[b][0] + part[b][1]) + (part[b][2] + part[b][3]);
+}
+
+// chunk_compute for NB vectors: the chunk's indices and values stay in
+// registers while one vector after the other is gathered and summed; the sums
+// are those of chunk_compute.
+template <typename VT, typename T, int EPT, int NB, typename XG>
+__device__ __forceinline__ void chunk_compute_multi(const WaveChunk<VT, EPT>& C, const int* __restrict__ JA,
+                                                    const int* __restrict__ IA, const VT* __restrict__ vals, XG xg,
+                                                    T* slice, T (&out)[NB])
+{
+    const int lane = threadIdx.x & 63;
+    if (C.e - C.s > EPT * 64) {
+        chunk_rows<VT, T, NB>(C.r0, C.nr, JA, IA, vals, xg, out);
+        return;
+    }
+    const int a = C.rb - C.s, e = C.re - C.s;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        T xv[EPT];
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) {
+            const int k = C.s + lane + 64 * j;
+            xv[j] = (k < C.e) ? xg(b, C.col[j]) : T(0);
+        }
+#pragma unroll
+        for (int j = 0; j < EPT; ++j) {
+            const int k = C.s + lane + 64 * j;
+            if (k < C.e) slice[k - C.s] = Load<VT, T>::get(C.v, j) * xv[j];
+        }
+        __builtin_amdgcn_wave_barrier();  // as in chunk_compute
+        T acc = T(0);
+        if (lane < C.nr && a < e) {
+            acc = slice[a];
+            for (int k = a + 1; k < e; ++k) acc += slice[k];
+        }
+        out[b] = acc;
+        __builtin_amdgcn_wave_barrier();
     }
 }
 

@@ -1,0 +1,82 @@
+"""The CSR product of rows with more than 8 entries on average (windows of 512
+entries per 64 rows) and of several vectors with shared values, at the edges of
+the windows, chunks and groups; int32 exactly, floats against FP64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def matrix(lengths, cols, seed, dtype):
+    rng = np.random.default_rng(seed)
+    JA = np.zeros(len(lengths) + 1, np.int32)
+    JA[1:] = np.cumsum(lengths)
+    IA = rng.integers(0, cols, JA[-1]).astype(np.int32)
+    V = rng.integers(-50, 50, IA.size).astype(dtype) if dtype == np.int32 else rng.standard_normal(IA.size).astype(dtype)
+    return JA, IA, V
+
+
+def check(cm, lengths, cols, dtype, batches=1, mode=0, shared_x=False, seed=0):
+    JA, IA, V = matrix(lengths, cols, seed, dtype)
+    n = len(lengths)
+    rng = np.random.default_rng(seed + 1)
+    draw = (lambda m: rng.integers(-50, 50, m).astype(dtype)) if dtype == np.int32 else (
+        lambda m: rng.standard_normal(m).astype(dtype))
+    x, y = draw((1 if shared_x else batches) * cols), draw(batches * n)
+    A = cm.SparseMatrix.from_csr(n, cols, JA, IA, V)
+    Y = cm.DeviceArray.from_numpy(y, rows=n, batches=batches)
+    X = cm.DeviceArray.from_numpy(x, rows=cols, batches=1 if shared_x else batches)
+    A.matvec(X, out=Y, mode=mode)
+    got = Y.numpy().reshape(batches, n)
+    wide = np.int64 if dtype == np.int32 else np.float64
+    rows = np.repeat(np.arange(n), np.diff(JA))
+    for b in range(batches):
+        terms = V.astype(wide) * x.reshape(-1, cols)[0 if shared_x else b].astype(wide)[IA]
+        total, size = np.zeros(n, wide), np.zeros(n, wide)
+        np.add.at(total, rows, terms)
+        np.add.at(size, rows, np.abs(terms))
+        base = y.reshape(batches, n)[b].astype(wide) * (mode == 1)
+        if dtype == np.int32:
+            assert np.array_equal(got[b], (total + base).astype(np.int32))
+        else:
+            # every term meets at most its row's length additions and one product rounding
+            bound = np.finfo(dtype).eps * ((np.asarray(lengths) + 2) * size + np.abs(base))
+            assert np.all(np.abs(got[b] - (total + base)) <= bound)
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 1000])
+@pytest.mark.parametrize("length", [9, 27, 32, 64, 127, 128, 129, 700])
+def test_row_lengths(gpu, rows, length):
+    check(gpu, [length] * rows, 5000, np.int32)
+    check(gpu, [length] * rows, 5000, np.float32, mode=gpu.capi.ADD)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.float32, np.float64])
+def test_ragged_rows(gpu, dtype):
+    rng = np.random.default_rng(3)
+    lengths = rng.integers(0, 60, 4321)
+    lengths[1000:1100] = 0
+    lengths[2000] = 5000  # its chunk goes row by row
+    check(gpu, lengths, 9000, dtype)
+
+
+@pytest.mark.parametrize("batches", [2, 3, 4, 5, 8])
+@pytest.mark.parametrize("mean", [4, 12])
+def test_vectors_together(gpu, batches, mean):
+    rows = 64 * 16384 // batches + 17  # past the rule: groups of vectors
+    lengths = np.random.default_rng(batches).integers(0, 2 * mean + 1, rows)
+    check(gpu, lengths, 1000, np.int32 if batches % 2 else np.float32, batches=batches)
+
+
+def test_shared_vector_and_bf16_values(gpu):
+    cm = gpu
+    check(cm, [20] * 3000, 3000, np.float32, batches=3, shared_x=False)
+    JA, IA, V = matrix([20] * 3000, 3000, 5, np.float32)
+    bits = (V.view(np.uint32) >> 16).astype(np.uint16)  # truncated to bf16
+    A = cm.SparseMatrix(cm.SparsityPattern(3000, 3000, JA, IA), cm.DeviceArray.from_numpy(bits))
+    x = np.random.default_rng(6).integers(-8, 8, 3000).astype(np.float32)
+    got = A.matvec(cm.DeviceArray.from_numpy(x)).numpy()
+    v = (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    terms = v * x[IA]
+    want, size = (np.add.reduceat(t, JA[:-1]) for t in (terms, np.abs(terms)))
+    assert np.all(np.abs(got - want) <= 2.0 ** -23 * 22 * size)
