@@ -808,6 +808,146 @@ __global__ __launch_bounds__(CG_BS) void cg_iter_kernel(int n, int it, int B, in
     if (threadIdx.x == 0) part1[(long long)bb * gridDim.x + blockIdx.x] = s;
 }
 
+// KA over the diagonals (cg_dia.hpp), it >= 1: the evaluation of cg_iter_kernel,
+// then p_it and Ap_it of one row per thread, p_it recomputed at each of the
+// row's columns from r, M^-1 and p_{it-1}. At these sizes (up to 2^17 unknowns)
+// the launch is a chain of memory latencies: the CSR form waits for the state,
+// the row bounds, the entries and the gathers in turn. Here everything but
+// the evaluation's partials has a known address, so the first rows' loads and
+// the state are requested together, before the state is looked at.
+// Measured on MI355X, us per launch at 128^2 FP32: 5.9 -> 3.8 (an empty launch
+// is 2 to 3 of them); whole iterations 9.9 -> 8.1, 360^2 10.8 -> 8.8, FP64 128^2
+// 11.3 -> 9.0, 8 right-hand sides of 128^2 13.1 -> 9.5. One element per thread in
+// KB (four times the blocks) changed nothing.
+template <typename VT, typename T, int D>
+__global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B, int G2, const DiaArgs A,
+                                                            const VT* __restrict__ dia, const T* __restrict__ invd,
+                                                            int istride, const T* __restrict__ r,
+                                                            const T* __restrict__ pprev, T* __restrict__ pnext,
+                                                            T* __restrict__ tmp, T* __restrict__ part1,
+                                                            const T* __restrict__ part2, CgState<T>* st,
+                                                            const T* __restrict__ diag, CgMirror* __restrict__ mirror)
+{
+    const int bb = blockIdx.y;
+    __shared__ T red[2 * CG_BS / 64];
+    __shared__ T rr_s[CG_MAXB], rz_s[CG_MAXB];
+    __shared__ T pairs[2 * CG_BS];
+    __shared__ T q_s[CG_MAXB];
+    const int lane = threadIdx.x & 63;
+    const long long off = (long long)bb * n;
+    const VT* db = dia + bb * A.bstride;
+    const T* ib = invd + (long long)bb * istride;
+    const T* rb = r + off;
+    const T* pp = pprev + off;
+    RowBlockWalk w(blockIdx.x, gridDim.x, div_up_dev(n, CG_BS));
+    T val[D], po[D], ro[D], io[D], pw = T(0), rw = T(0), iw = T(0);
+    auto load = [&]() {
+        const long long row = min((long long)w.cur * CG_BS + threadIdx.x, (long long)n - 1);
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            // a slot the row does not store holds 0: any column of this vector will do
+            const long long c = min(max(row + A.off[d], 0ll), (long long)n - 1);
+            val[d] = dia_value<VT, T>(db[d * A.ld + row]);
+            po[d] = pp[c];
+            ro[d] = rb[c];
+            io[d] = ib[c];
+        }
+        pw = pp[row];
+        rw = rb[row];
+        iw = ib[row];
+    };
+    if (w.valid()) load();
+    // ---- the state and the previous iteration's sums (as cg_iter_kernel)
+    const int status = st->status;
+    const bool per_batch = st->per_batch != 0;
+    const int done_k = (lane < B && per_batch) ? st->bdone[lane] : (int)CG_RUNNING;
+    const T thr_k = lane < B ? st->thr[lane] : T(0);
+    const T rhs_k = lane < B ? st->rhs2[lane] : T(1);
+    const T thr_own = st->thr[bb];
+    const int max_iter = st->max_iter;
+    const int own_done = per_batch ? st->bdone[bb] : (int)CG_RUNNING;
+    const int prev = it - 1;
+    const T absOld = st->absNew[prev & 1][bb];
+    if (B == 1) {
+        T a, c;
+        reduce_partials_pair(part2, G2, a, c, red);
+        if (threadIdx.x == 0) { rr_s[0] = a; rz_s[0] = c; }
+    } else if (B <= CG_WAVE_FOLD_B) {
+        reduce_batched_waves(part1, 0, part2, G2, B, rr_s, rz_s, red);
+    } else {
+        reduce_pairs_batched(part2, G2, B, rr_s, rz_s, pairs);
+    }
+    __syncthreads();
+    if (status != CG_RUNNING) return;
+    const bool own_prev = own_done != CG_RUNNING;
+    // a batch that finished earlier has nothing to do; block (0,0) still
+    // evaluates, it owns the global status
+    if (own_prev && !(blockIdx.x == 0 && bb == 0)) return;
+    const bool all = __ballot(lane < B && done_k == CG_RUNNING && !(rr_s[lane] < thr_k)) == 0;
+    const bool own_conv = own_prev || rr_s[bb] < thr_own;
+    if (threadIdx.x < B) q_s[lane] = rr_s[lane] / rhs_k;  // read below by thread 0, in this wavefront
+    __builtin_amdgcn_wave_barrier();
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (per_batch && !own_prev) {
+            st->berr[bb] = sqrt((double)q_s[bb]);
+            if (own_conv) {
+                st->bdone[bb] = CG_CONVERGED;
+                st->biters[bb] = prev;  // the converging step is not counted
+            } else {
+                st->biters[bb] = it;
+            }
+        }
+        const bool pub = all || it >= max_iter || (prev % CG_CHUNK) == CG_CHUNK - 1;
+        if (per_batch && !own_prev && (pub || own_conv)) {
+            mirror->berr[bb] = st->berr[bb];
+            mirror->biters[bb] = st->biters[bb];
+            mirror->bdone[bb] = st->bdone[bb];
+        }
+        if (bb == 0) {
+            if (!per_batch) {
+                T m = 0;
+                for (int k = 0; k < B; ++k) m = (k == 0 || q_s[k] > m) ? q_s[k] : m;
+                st->err = sqrt((double)m);
+            }
+            if (all) {
+                st->status = CG_CONVERGED;
+                st->iters = prev;
+            } else {
+                st->iters = it;
+                if (it >= max_iter) st->status = CG_MAXIT;
+            }
+            if (pub) {
+                mirror->err = st->err;
+                mirror->iters = st->iters;
+                mirror->it_done = prev;
+                mirror->status = st->status;
+            }
+        }
+        if (!(per_batch && own_conv)) st->absNew[it & 1][bb] = rz_s[bb];
+    }
+    if (per_batch ? own_conv : all) return;
+    if (it >= max_iter) return;
+    const T beta = rz_s[bb] / absOld;
+    T s = T(0);
+    while (w.valid()) {
+        const long long row = (long long)w.cur * CG_BS + threadIdx.x;
+        if (row < n) {
+            T ap = val[0] * cg_pnext(beta, po[0], io[0], ro[0]);
+#pragma unroll
+            for (int d = 1; d < D; ++d) ap += val[d] * cg_pnext(beta, po[d], io[d], ro[d]);
+            const T pv = cg_pnext(beta, pw, iw, rw);
+            if (diag) ap += diag[row] * pv;
+            pnext[off + row] = pv;
+            tmp[off + row] = ap;
+            s += pv * ap;
+        }
+        w.next();
+        if (w.valid()) load();
+    }
+    s = block_reduce<OpSum, CG_BS>(s, red);
+    if (threadIdx.x == 0) part1[(long long)bb * gridDim.x + blockIdx.x] = s;
+}
+
 // Vector width of K2 / K3: VW elements per load (VW = 16 / sizeof(T) when n
 // is a multiple of it and every vector is 16-byte aligned, else 1).
 // loads / stores of a vector stream, non-temporal (streaming) when NT
@@ -841,7 +981,9 @@ __device__ __forceinline__ T cg_hsum(const typename CgVec<T, VW>::type& v)
 // reads p anyway, so this pass reads r, Ap, M^-1 and writes r only.
 // VNT: streams loaded / stored non-temporally (bit 0 r, 1 tmp, 2 M^-1,
 // 3 the r store)
-template <typename T, bool UPDATE_X, int VW = 1, int VNT = 0>
+// EAGER: the state is looked at after the loads and the partials' fold instead
+// of before (one memory latency less where the launch is nothing else).
+template <typename T, bool UPDATE_X, int VW = 1, int VNT = 0, bool EAGER = false>
 __global__ __launch_bounds__(CG_BS) void cg_update_kernel(int n, int it_arg, int G1, const T* __restrict__ part1,
                                                           const T* __restrict__ invd, int istride,
                                                           const T* __restrict__ p, const T* __restrict__ tmp,
@@ -853,7 +995,9 @@ __global__ __launch_bounds__(CG_BS) void cg_update_kernel(int n, int it_arg, int
     // the setup then does not write r)
     typedef typename CgVec<T, VW>::type V;
     const int bb = blockIdx.y;
-    if (batch_inactive(st, bb)) return;
+    if (!EAGER && batch_inactive(st, bb)) return;
+    const int e_status = EAGER ? st->status : (int)CG_RUNNING;
+    const int e_done = (EAGER && st->per_batch) ? st->bdone[bb] : (int)CG_RUNNING;
     const int it = it_arg >= 0 ? it_arg : st->it;  // < 0: the counter kept by K1
     __shared__ T red[2 * CG_BS / 64];
     const long long off = (long long)bb * n;
@@ -886,6 +1030,7 @@ __global__ __launch_bounds__(CG_BS) void cg_update_kernel(int n, int it_arg, int
     const T rz = st->absNew[it & 1][bb];
     load(i0);
     const T pap = reduce_partials(part1 + (long long)bb * G1, G1, 1, red);
+    if (EAGER && (e_status != CG_RUNNING || e_done != CG_RUNNING)) return;
     const T alpha = rz / pap;
     V vrr = V(0), vrz = V(0);
     while (i0 < nv) {
@@ -1202,6 +1347,24 @@ struct CgBatchOpts {
     const BlockOp* block = nullptr;  // a block-CSR operator replaces the CSR matrix (FP32)
 };
 
+// The diagonals the two-launch form is built for (a row's operands stay in
+// registers).
+inline bool cg_dia_iter_takes(int count) { return count == 3 || count == 5 || count == 7; }
+
+template <typename VT, typename T>
+static void launch_cg_dia_iter(hipStream_t stream, int n, int it, int B, int G1, int G2, const DiaArgs& A,
+                               const VT* dia, const T* invd, int istride, const T* r, const T* pprev, T* pnext, T* tmp,
+                               T* part1, const T* part2, CgState<T>* st, const T* diag, CgMirror* mirror)
+{
+#define CM_DIA_ITER(D)                                                                                      \
+    cg_dia_iter_kernel<VT, T, D><<<dim3(G1, B), CG_BS, 0, stream>>>(n, it, B, G2, A, dia, invd, istride, r, \
+                                                                    pprev, pnext, tmp, part1, part2, st, diag, mirror)
+    if (A.count == 3) CM_DIA_ITER(3);
+    else if (A.count == 5) CM_DIA_ITER(5);
+    else CM_DIA_ITER(7);
+#undef CM_DIA_ITER
+}
+
 // Queues the layout by diagonals; *dia stays NULL where it does not pay or
 // no memory is left (the solve then keeps the CSR product).
 template <typename VT>
@@ -1369,7 +1532,7 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     int it = 0;
     // K1 over the diagonals (cg_dia.hpp): laid out after the first chunk if
     // enough iterations are left to pay for it, used from CG_DIA_FROM on
-    const bool try_dia = !fused && !dense && !block && max_iter >= CG_DIA_FROM + 2 * CG_CHUNK && nnz > 0;
+    const bool try_dia = !dense && !block && max_iter >= CG_DIA_FROM + 2 * CG_CHUNK && nnz > 0;
     const long long dia_ld = ((long long)n + 7) / 8 * 8;
     DiaArgs da{};
     VT* dia = nullptr;
@@ -1384,8 +1547,12 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
             da.ld = dia_ld;
             da.bstride = vstride ? da.count * dia_ld : 0;
             for (int d = 0; d < da.count; ++d) da.off[d] = hplan->off[d];
+            if (fused && !cg_dia_iter_takes(da.count)) {
+                dia = nullptr;
+                continue;
+            }
             dia_on = &da;
-            G1 = walk_grid(div_up(n, cg_dia_rows_per_block(n)), gcap);
+            if (!fused) G1 = walk_grid(div_up(n, cg_dia_rows_per_block(n)), gcap);
         }
         for (int k = 0; k < todo; ++k, ++it) {
             if (!fused) {
@@ -1394,6 +1561,13 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
                 continue;
             }
             T* pcur = pbuf[it & 1];
+            if (dia_on) {
+                launch_cg_dia_iter<VT, T>(ctx->stream, n, it, B, G1, G2, da, dia, invd, istride, r, pbuf[(it - 1) & 1],
+                                          pcur, t, part1, part2, st, diag, mirror);
+                cg_update_kernel<T, true, 1, 0, true><<<dim3(G2, B), CG_BS, 0, ctx->stream>>>(
+                    n, it, G1, part1, invd, istride, pcur, t, x, r, part2, st, r0);
+                continue;
+            }
             if (it == 0)
                 cg_iter_kernel<VT, T, true><<<dim3(G1, B), CG_BS, 0, ctx->stream>>>(
                     n, it, B, G2, JA, IA, vals, vstride, invd, istride, r, pcur, pcur, t, part1, part2, st, diag,
