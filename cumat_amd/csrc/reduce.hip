@@ -18,6 +18,7 @@
 // Every combination order is fixed, so results are bit-reproducible.
 #include "cm_common.hpp"
 
+#include <algorithm>
 #include <limits>
 
 // Fixed device buffer of cm_dot_noalloc: the per-chunk partial sums of one
@@ -240,18 +241,101 @@ __global__ __launch_bounds__(RBS) void col_kernel(const S* __restrict__ in, long
     if (w == 0) partials[(long long)blockIdx.x * 64 + threadIdx.x] = acc;
 }
 
-// Folds the ksplit partial rows of every (p, q-tile) in split order.
-template <typename Op, typename T, typename S>
-__global__ __launch_bounds__(64) void col_combine_kernel(const T* __restrict__ partials, long long Q, int ksplit,
-                                                         S* out)
+// Folds the ksplit partial rows of every (p, q-tile): the block's wavefronts
+// take every NW-th of them in split order, four loads in flight, and are
+// combined in order. (One wavefront folding them one after the other took most
+// of a long fold's time: 1024 x 1024 x 64 FP32 over columns and batches, 512
+// partials a tile, 164 -> 52 us; 51 x 20001 x 10 249 -> 16.)
+template <typename Op, typename T, typename S, int NW>
+__global__ __launch_bounds__(64 * NW) void col_combine_kernel(const T* __restrict__ partials, long long Q, int ksplit,
+                                                              S* out)
 {
+    __shared__ T lds[64 * NW];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const long long qtiles = (Q + 63) / 64;
     const long long tile = blockIdx.x;
     const long long p = tile / qtiles;
-    const long long q = (tile % qtiles) * 64 + threadIdx.x;
+    const long long q = (tile % qtiles) * 64 + lane;
+    const T* pt = partials + tile * ksplit * 64 + lane;
     T r = Identity<Op, T>::v();
-    for (int k2 = 0; k2 < ksplit; ++k2) r = Op::apply(r, partials[(tile * ksplit + k2) * 64 + threadIdx.x]);
-    if (q < Q) out[p * Q + q] = (S)r;
+    int k = w;
+    for (; k + 3 * NW < ksplit; k += 4 * NW) {
+        const T v0 = pt[k * 64], v1 = pt[(k + NW) * 64], v2 = pt[(k + 2 * NW) * 64], v3 = pt[(k + 3 * NW) * 64];
+        r = Op::apply(r, Op::apply(Op::apply(v0, v1), Op::apply(v2, v3)));
+    }
+    for (; k < ksplit; k += NW) r = Op::apply(r, pt[k * 64]);
+    lds[threadIdx.x] = r;
+    __syncthreads();
+    if (w != 0 || q >= Q) return;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) r = Op::apply(r, lds[64 * i + lane]);
+    out[p * Q + q] = (S)r;
+}
+
+// Few kept elements (Q <= COL_NARROW): a wavefront takes 64 / Q consecutive
+// rows at once, lane = row * Q + q, so most lanes work; the rows' results are
+// combined in LDS in order. Lanes of col_kernel beyond Q idle: 8 x 60000 x 64
+// FP32 over columns 161 -> 25 us, over columns and batches 375 -> 28.
+constexpr int COL_NARROW = 32;
+template <typename Op, typename T, typename S>
+__global__ __launch_bounds__(RBS) void col_narrow_kernel(const S* __restrict__ in, int Q, long long K, long long st,
+                                                         long long PS, int ksplit, T* partials, S* out)
+{
+    __shared__ T lds[RBS];
+    constexpr int NW = RBS / 64;
+    const int per = 64 / Q;  // rows per wavefront and step
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int sub = lane / Q, q = lane - sub * Q;
+    const long long p = blockIdx.x / ksplit;
+    const int ks = blockIdx.x % ksplit;
+    const long long kchunk = (K + ksplit - 1) / ksplit;
+    const long long kb = ks * kchunk, ke = min(K, kb + kchunk);
+    const long long step = (long long)NW * per;
+    T acc = Identity<Op, T>::v();
+    if (sub < per) {
+        const S* col = in + p * PS + q;
+        long long k = kb + w * per + sub;
+        for (; k + 3 * step < ke; k += 4 * step) {
+            const T v0 = (T)col[k * st], v1 = (T)col[(k + step) * st], v2 = (T)col[(k + 2 * step) * st],
+                    v3 = (T)col[(k + 3 * step) * st];
+            acc = Op::apply(acc, Op::apply(Op::apply(v0, v1), Op::apply(v2, v3)));
+        }
+        for (; k < ke; k += step) acc = Op::apply(acc, (T)col[k * st]);
+    }
+    lds[threadIdx.x] = acc;
+    __syncthreads();
+    if ((int)threadIdx.x >= Q) return;
+    T r = lds[threadIdx.x];
+    for (int i = 1; i < NW * per; ++i) r = Op::apply(r, lds[i / per * 64 + i % per * Q + threadIdx.x]);
+    if (ksplit == 1) out[p * Q + threadIdx.x] = (S)r;
+    else partials[(long long)blockIdx.x * 64 + threadIdx.x] = r;
+}
+
+// Short folds (K < 256) over many kept elements that col_stream_v4_kernel
+// cannot take (odd sizes, 8-byte and 1-byte types): a thread per output, eight
+// rows in flight, folded in order. With the block's wavefronts splitting K, as
+// in col_kernel, a fold of 3 rows leaves one of four at work: 3001 x 5003 x 3
+// FP32 over batches 195 -> 71 us, 51 x 20001 x 10 18 -> 10.
+template <typename Op, typename T, typename S>
+__global__ __launch_bounds__(RBS) void col_short_kernel(const S* __restrict__ in, long long PQ, long long Q,
+                                                        long long K, long long st, long long PS, S* out)
+{
+    constexpr int U = 8;
+    const long long i = (long long)blockIdx.x * RBS + threadIdx.x;
+    if (i >= PQ) return;
+    const long long p = i / Q, q = i - p * Q;
+    const S* col = in + p * PS + q;
+    T acc = Identity<Op, T>::v();
+    long long k = 0;
+    for (; k + U <= K; k += U) {
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = (T)col[(k + u) * st];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = Op::apply(acc, v[u]);
+    }
+    for (; k < K; ++k) acc = Op::apply(acc, (T)col[k * st]);
+    out[i] = (S)acc;
 }
 
 // col_kernel with 16-byte loads (4-byte types, Q, st and PS multiples of 4,
@@ -370,27 +454,40 @@ __global__ __launch_bounds__(RBS) void col_stream_v4_kernel(const T* __restrict_
         if (ok[u]) *(reinterpret_cast<T4*>(out + p * Q) + q40 + u * RBS) = acc[u];
 }
 
-// Folds the ksplit partial tiles of col_kernel_v4 in split order.
-template <typename Op, typename T>
-__global__ __launch_bounds__(64) void col_combine_v4_kernel(const T* __restrict__ partials, long long Q, int ksplit,
-                                                            T* out)
+// Folds the ksplit partial tiles of col_kernel_v4 (as col_combine_kernel).
+template <typename Op, typename T, int NW>
+__global__ __launch_bounds__(64 * NW) void col_combine_v4_kernel(const T* __restrict__ partials, long long Q,
+                                                                 int ksplit, T* out)
 {
     typedef T T4 __attribute__((ext_vector_type(4)));
+    __shared__ T4 lds[64 * NW];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const long long Q4 = Q / 4;
     const long long qtiles = (Q4 + 63) / 64;
     const long long tile = blockIdx.x;
     const long long p = tile / qtiles;
-    const long long q4 = (tile % qtiles) * 64 + threadIdx.x;
-    const T4* pt = reinterpret_cast<const T4*>(partials);
-    T4 r = pt[(tile * ksplit) * 64 + threadIdx.x];
-    for (int k2 = 1; k2 < ksplit; ++k2) {
-        const T4 v = pt[(tile * ksplit + k2) * 64 + threadIdx.x];
-        r.x = Op::apply(r.x, v.x);
-        r.y = Op::apply(r.y, v.y);
-        r.z = Op::apply(r.z, v.z);
-        r.w = Op::apply(r.w, v.w);
-    }
-    if (q4 < Q4) *(reinterpret_cast<T4*>(out + p * Q) + q4) = r;
+    const long long q4 = (tile % qtiles) * 64 + lane;
+    const T4* pt = reinterpret_cast<const T4*>(partials) + tile * ksplit * 64 + lane;
+    auto app = [](T4 a, T4 b) {
+        T4 r;
+        r.x = Op::apply(a.x, b.x);
+        r.y = Op::apply(a.y, b.y);
+        r.z = Op::apply(a.z, b.z);
+        r.w = Op::apply(a.w, b.w);
+        return r;
+    };
+    const T id = Identity<Op, T>::v();
+    T4 r = {id, id, id, id};
+    int k = w;
+    for (; k + 3 * NW < ksplit; k += 4 * NW)
+        r = app(r, app(app(pt[k * 64], pt[(k + NW) * 64]), app(pt[(k + 2 * NW) * 64], pt[(k + 3 * NW) * 64])));
+    for (; k < ksplit; k += NW) r = app(r, pt[k * 64]);
+    lds[threadIdx.x] = r;
+    __syncthreads();
+    if (w != 0 || q4 >= Q4) return;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) r = app(r, lds[64 * i + lane]);
+    *(reinterpret_cast<T4*>(out + p * Q) + q4) = r;
 }
 
 // ------------------------------------------ 16-byte block-per-chunk path
@@ -566,12 +663,38 @@ static int run_segments(cm_ctx_t ctx, Src src, long long L, long long nseg, S* o
 }
 
 template <typename Op, typename T, typename S>
+static int combine_columns(cm_ctx_t ctx, const T* part, long long tiles, long long Q, int ksplit, S* out)
+{
+    // enough wavefronts for a handful of partials each
+    if (ksplit >= 64)
+        col_combine_kernel<Op, T, S, 16><<<(unsigned)tiles, 1024, 0, ctx->stream>>>(part, Q, ksplit, out);
+    else
+        col_combine_kernel<Op, T, S, 4><<<(unsigned)tiles, 256, 0, ctx->stream>>>(part, Q, ksplit, out);
+    CM_LAUNCH_CHECK();
+    return CM_OK;
+}
+
+template <typename Op, typename T, typename S>
 static int run_columns(cm_ctx_t ctx, const S* in, long long P, long long Q, long long K, long long st,
                        long long PS, S* out)
 {
     if (P * Q == 0) return CM_OK;
     if (K == 0) return fail(CM_E_DIM, "reduction over an empty axis");
     const long long cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    // few kept elements and a fold of several steps of a block
+    if (Q <= COL_NARROW && K >= 64) {
+        const long long per = 64 / Q;
+        long long ksplit = std::max<long long>(1, (cus * 8 + P - 1) / P);
+        ksplit = std::max<long long>(1, std::min<long long>({ksplit, K / (16 * per), 1024}));
+        void* part = nullptr;
+        if (ksplit > 1) CM_TRY(scratch(ctx, 1, sizeof(T) * P * ksplit * 64, &part));
+        CM_REQUIRE(P * ksplit < (1ll << 31), CM_E_DIM, "reduction too large");
+        col_narrow_kernel<Op, T, S><<<(unsigned)(P * ksplit), RBS, 0, ctx->stream>>>(in, (int)Q, K, st, PS,
+                                                                                     (int)ksplit, (T*)part, out);
+        CM_LAUNCH_CHECK();
+        if (ksplit > 1) CM_TRY((combine_columns<Op, T, S>(ctx, (const T*)part, P, Q, (int)ksplit, out)));
+        return CM_OK;
+    }
     if constexpr (std::is_same<S, T>::value && sizeof(T) == 4) {
         const bool aligned = Q % 4 == 0 && st % 4 == 0 && PS % 4 == 0 && (((uintptr_t)in & 15) == 0) &&
                              (((uintptr_t)out & 15) == 0);
@@ -622,12 +745,25 @@ static int run_columns(cm_ctx_t ctx, const S* in, long long P, long long Q, long
                                                                              (int)ksplit, (T*)part, (T*)out);
             CM_LAUNCH_CHECK();
             if (ksplit > 1) {
-                col_combine_v4_kernel<Op, T><<<(unsigned)tiles, 64, 0, ctx->stream>>>((const T*)part, Q, (int)ksplit,
-                                                                                      (T*)out);
+                // enough wavefronts for a handful of partials each
+                if (ksplit >= 64)
+                    col_combine_v4_kernel<Op, T, 16><<<(unsigned)tiles, 1024, 0, ctx->stream>>>((const T*)part, Q,
+                                                                                               (int)ksplit, (T*)out);
+                else
+                    col_combine_v4_kernel<Op, T, 4><<<(unsigned)tiles, 256, 0, ctx->stream>>>((const T*)part, Q,
+                                                                                             (int)ksplit, (T*)out);
                 CM_LAUNCH_CHECK();
             }
             return CM_OK;
         }
+    }
+    // short folds, a thread per output where that fills the chip
+    if (K < 256 && P * Q >= cus * 1024) {
+        const long long blocks = (P * Q + RBS - 1) / RBS;
+        CM_REQUIRE(blocks < (1ll << 31), CM_E_DIM, "reduction too large");
+        col_short_kernel<Op, T, S><<<(unsigned)blocks, RBS, 0, ctx->stream>>>(in, P * Q, Q, K, st, PS, out);
+        CM_LAUNCH_CHECK();
+        return CM_OK;
     }
     long long tiles = P * ((Q + 63) / 64);
     long long ksplit = 1;
@@ -646,8 +782,7 @@ static int run_columns(cm_ctx_t ctx, const S* in, long long P, long long Q, long
                                                                       out);
     CM_LAUNCH_CHECK();
     if (ksplit > 1) {
-        col_combine_kernel<Op, T, S><<<(unsigned)tiles, 64, 0, ctx->stream>>>((const T*)part, Q, (int)ksplit, out);
-        CM_LAUNCH_CHECK();
+        CM_TRY((combine_columns<Op, T, S>(ctx, (const T*)part, tiles, Q, (int)ksplit, out)));
     }
     return CM_OK;
 }

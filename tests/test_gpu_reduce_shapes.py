@@ -1,0 +1,59 @@
+"""Reductions of stored arrays whose kept axis is the contiguous one, at the
+shapes where the kernels change: few kept elements (several rows per wavefront),
+short folds (a thread per output), long folds with many partials; all types."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [np.float32, np.float64, np.int32, np.bool_]
+
+
+def check(cm, shape, axis, dtype, op="sum"):
+    B, R, C = shape
+    rng = np.random.default_rng(R + C + B)
+    if dtype == np.bool_:
+        a, op = rng.uniform(size=shape) < 0.999, "all"
+    elif dtype == np.int32:
+        a = rng.integers(-1000, 1000, shape).astype(dtype)
+    else:
+        a = rng.uniform(0, 1, shape).astype(dtype)
+    got = cm.reduce(cm.DeviceArray.from_numpy(a), op, axis).numpy(logical=True)
+    dims = tuple(d for d, bit in ((1, 1), (2, 2), (0, 4)) if axis & bit)
+    if dtype == np.bool_:
+        assert np.array_equal(got, a.all(axis=dims, keepdims=True))
+    elif dtype == np.int32:
+        f = {"sum": np.sum, "min": np.min, "max": np.max}[op]
+        assert np.array_equal(got, f(a.astype(np.int64), axis=dims, keepdims=True).astype(np.int32))
+    else:
+        want = a.astype(np.float64).sum(axis=dims, keepdims=True)
+        n = a.size / want.size
+        # positive terms: a chain of at most 2048 of them, then trees
+        assert np.all(np.abs(got - want) <= np.finfo(dtype).eps * (min(n, 2048) + 30) * want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [2, 3, 8, 31, 32, 33])
+@pytest.mark.parametrize("cols", [63, 64, 65, 1000, 70001])
+def test_few_kept_elements(gpu, dtype, rows, cols):
+    check(gpu, (1, rows, cols), 2, dtype)
+    check(gpu, (5, rows, cols // 5), 2, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batches", [2, 3, 7, 8, 9, 61])
+def test_short_folds(gpu, dtype, batches):
+    check(gpu, (batches, 517, 519), 4, dtype)  # one output more than a thread each for 256 CUs x 1024
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(40, 100, 700), (40, 1024, 257), (7, 64, 5003), (3, 260, 9001)])
+def test_long_folds(gpu, dtype, shape):
+    check(gpu, shape, 6, dtype)
+    check(gpu, shape, 2, dtype)
+
+
+@pytest.mark.parametrize("op", ["min", "max"])
+def test_extrema(gpu, op):
+    for shape, axis in (((1, 5, 9000), 2), ((3, 600, 601), 4), ((9, 100, 900), 6)):
+        check(gpu, shape, axis, np.int32, op)
