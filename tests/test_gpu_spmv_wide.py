@@ -80,3 +80,21 @@ def test_shared_vector_and_bf16_values(gpu):
     terms = v * x[IA]
     want, size = (np.add.reduceat(t, JA[:-1]) for t in (terms, np.abs(terms)))
     assert np.all(np.abs(got - want) <= 2.0 ** -23 * 22 * size)
+
+
+@pytest.mark.parametrize("batches", [1, 2, 3, 5])
+@pytest.mark.parametrize("width", [3, 8, 9, 27])
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+def test_ell_vectors_together(gpu, batches, width, dtype):
+    """ELLPACK with padding, past the rule for groups of vectors: integer data, exact in every type."""
+    cm = gpu
+    rows, cols = 64 * 16384 // batches + 5, 777
+    rng = np.random.default_rng(width)
+    idx = rng.integers(-1, cols, (rows, width)).astype(np.int32)
+    val = rng.integers(-9, 10, (rows, width)).astype(dtype)
+    x = rng.integers(-9, 10, (batches, cols)).astype(dtype)
+    A = cm.ELLMatrix(rows, cols, idx, val)
+    got = A.matvec(cm.DeviceArray.from_numpy(x.reshape(-1), rows=cols, batches=batches)).numpy().reshape(batches, rows)
+    for b in range(batches):
+        want = np.where(idx >= 0, val * x[b][np.maximum(idx, 0)], 0).sum(axis=1)
+        assert np.array_equal(got[b], want.astype(dtype))
