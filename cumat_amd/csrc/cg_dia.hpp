@@ -31,6 +31,11 @@
 namespace cm {
 
 constexpr int CG_DIA_MAX = 32;     // diagonals
+// Unknowns (n x batches) from which the three-launch form takes the layout:
+// below, an iteration is three launches whatever K1 reads, and the layout's 40
+// us stay (32^2 13.4 us per iteration without, 13.6 with, 200 iterations; two
+// systems of 48^2 15.2 and 13.6).
+constexpr long long CG_DIA_MIN = 2048;
 constexpr int CG_DIA_SAMPLE = 2048;  // rows the detection looks at
 constexpr int CG_DIA_DETECT_BS = 1024;
 constexpr int CG_DIA_BS = 256;

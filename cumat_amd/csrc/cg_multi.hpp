@@ -1532,7 +1532,7 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     int it = 0;
     // K1 over the diagonals (cg_dia.hpp): laid out after the first chunk if
     // enough iterations are left to pay for it, used from CG_DIA_FROM on
-    const bool try_dia = !dense && !block && max_iter >= CG_DIA_FROM + 2 * CG_CHUNK && nnz > 0;
+    const bool try_dia = !dense && !block && (fused || N >= CG_DIA_MIN) && max_iter >= CG_DIA_FROM + 2 * CG_CHUNK && nnz > 0;
     const long long dia_ld = ((long long)n + 7) / 8 * 8;
     DiaArgs da{};
     VT* dia = nullptr;

@@ -54,7 +54,7 @@ def check(cm, orc, JA, IA, V, rhs=1, dtype=np.float32, tol=1e-5):
         assert np.linalg.norm(bk - y) / np.linalg.norm(bk) <= bound
 
 
-@pytest.mark.parametrize("n", [255, 256, 513, 1023, 4099, 70001])
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 2559, 2560, 2561, 70001])
 @pytest.mark.parametrize("offsets", [(1,), (1, 37), (1, 5, 31), (1, 2, 3, 4, 5, 11, 12, 13, 40, 41, 42, 43, 44)])
 def test_diagonals(gpu, orc, n, offsets):
     check(gpu, orc, *banded(n, offsets, n))
@@ -71,7 +71,7 @@ def test_four_rows_per_lane(gpu, orc):
 
 
 def test_too_many_diagonals(gpu, orc):
-    check(gpu, orc, *banded(2000, tuple(range(1, 34, 2)), 4))  # 35 diagonals
+    check(gpu, orc, *banded(2600, tuple(range(1, 34, 2)), 4))  # 35 diagonals
 
 
 def test_columns_out_of_order(gpu, orc):
@@ -98,7 +98,7 @@ def test_entry_outside_the_sample(gpu, orc):
     check(gpu, orc, JA2, cols[order].astype(np.int32), vals[order])
 
 
-@pytest.mark.parametrize("batches", [1, 5])
+@pytest.mark.parametrize("batches", [2, 5])
 def test_values_per_batch(gpu, orc, batches):
     import torch
     from cumat_amd.problems import grid_laplacian, lognormal_sampler
