@@ -312,30 +312,56 @@ __global__ __launch_bounds__(RBS) void col_narrow_kernel(const S* __restrict__ i
 }
 
 // Short folds (K < 256) over many kept elements that col_stream_v4_kernel
-// cannot take (odd sizes, 8-byte and 1-byte types): a thread per output, eight
-// rows in flight, folded in order. With the block's wavefronts splitting K, as
-// in col_kernel, a fold of 3 rows leaves one of four at work: 3001 x 5003 x 3
-// FP32 over batches 195 -> 71 us, 51 x 20001 x 10 18 -> 10.
+// cannot take (odd sizes, 8-byte and 1-byte types): a thread per output, sixteen
+// rows in flight. With the block's wavefronts splitting K, as in col_kernel, a
+// fold of 3 rows leaves one of four at work. The thread keeps the four partials
+// that the wavefronts of col_kernel would hold and folds them in the same order,
+// so the results are bit-identical to it: one chain over the rows would lose up
+// to 4x in FP32 (255 uniform terms: rms error 1.79 eps of the sum against 0.41).
+// 3001 x 5003 x 3 FP32 over batches 224 -> 74 us, 51 x 20001 x 10 22 -> 14,
+// 517 x 519 x 200 50 -> 40 (col_kernel -> this).
 template <typename Op, typename T, typename S>
 __global__ __launch_bounds__(RBS) void col_short_kernel(const S* __restrict__ in, long long PQ, long long Q,
                                                         long long K, long long st, long long PS, S* out)
 {
-    constexpr int U = 8;
+    constexpr int NW = RBS / 64;
+    constexpr int U = 4 * NW;
     const long long i = (long long)blockIdx.x * RBS + threadIdx.x;
     if (i >= PQ) return;
     const long long p = i / Q, q = i - p * Q;
     const S* col = in + p * PS + q;
-    T acc = Identity<Op, T>::v();
+    T acc[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) acc[w] = Identity<Op, T>::v();
     long long k = 0;
     for (; k + U <= K; k += U) {
         T v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) v[u] = (T)col[(k + u) * st];
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc = Op::apply(acc, v[u]);
+        for (int w = 0; w < NW; ++w)
+            acc[w] = Op::apply(acc[w], Op::apply(Op::apply(v[w], v[w + NW]), Op::apply(v[w + 2 * NW], v[w + 3 * NW])));
     }
-    for (; k < K; ++k) acc = Op::apply(acc, (T)col[k * st]);
-    out[i] = (S)acc;
+    const int rest = (int)(K - k);
+    if (rest > 0) {
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = u < rest ? (T)col[(k + u) * st] : Identity<Op, T>::v();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            if (w + 3 * NW < rest) {
+                acc[w] = Op::apply(acc[w], Op::apply(Op::apply(v[w], v[w + NW]),
+                                                     Op::apply(v[w + 2 * NW], v[w + 3 * NW])));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    if (w + j * NW < rest) acc[w] = Op::apply(acc[w], v[w + j * NW]);
+            }
+        }
+    }
+#pragma unroll
+    for (int w = 1; w < NW; ++w) acc[0] = Op::apply(acc[0], acc[w]);
+    out[i] = (S)acc[0];
 }
 
 // col_kernel with 16-byte loads (4-byte types, Q, st and PS multiples of 4,

@@ -57,3 +57,31 @@ def test_long_folds(gpu, dtype, shape):
 def test_extrema(gpu, op):
     for shape, axis in (((1, 5, 9000), 2), ((3, 600, 601), 4), ((9, 100, 900), 6)):
         check(gpu, shape, axis, np.int32, op)
+
+
+def strided(x, k, step):
+    """A lane's fold of x[k], x[k + step], ...: groups of four, then one by one."""
+    acc = np.zeros_like(x[0])
+    while k + 3 * step < len(x):
+        acc = acc + ((x[k] + x[k + step]) + (x[k + 2 * step] + x[k + 3 * step]))
+        k += 4 * step
+    while k < len(x):
+        acc = acc + x[k]
+        k += step
+    return acc
+
+
+def chain(parts):
+    r = parts[0]
+    for v in parts[1:]:
+        r = r + v
+    return r
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("batches", [2, 3, 5, 8, 12, 13, 14, 15, 16, 17, 29, 32, 61, 100])
+def test_short_folds_keep_four_partials(gpu, dtype, batches):
+    # the order of four wavefronts splitting the fold, one output per thread
+    a = np.random.default_rng(batches).normal(size=(batches, 517, 519)).astype(dtype)
+    got = gpu.reduce(gpu.DeviceArray.from_numpy(a), "sum", 4).numpy(logical=True)
+    assert np.array_equal(got[0], chain([strided(a, w, 4) for w in range(4)]))
