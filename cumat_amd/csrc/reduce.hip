@@ -274,8 +274,8 @@ __global__ __launch_bounds__(64 * NW) void col_combine_kernel(const T* __restric
 
 // Few kept elements (Q <= COL_NARROW): a wavefront takes 64 / Q consecutive
 // rows at once, lane = row * Q + q, so most lanes work; the rows' results are
-// combined in LDS in order. Lanes of col_kernel beyond Q idle: 8 x 60000 x 64
-// FP32 over columns 161 -> 25 us, over columns and batches 375 -> 28.
+// combined in LDS by halves. Lanes of col_kernel beyond Q idle: 8 x 60000 x 64
+// FP32 over columns 162 -> 25 us, over columns and batches 376 -> 30.
 constexpr int COL_NARROW = 32;
 template <typename Op, typename T, typename S>
 __global__ __launch_bounds__(RBS) void col_narrow_kernel(const S* __restrict__ in, int Q, long long K, long long st,
@@ -304,9 +304,22 @@ __global__ __launch_bounds__(RBS) void col_narrow_kernel(const S* __restrict__ i
     }
     lds[threadIdx.x] = acc;
     __syncthreads();
+    // the wavefronts first, then the rows of one by halves: one chain over all
+    // of them (128 at Q = 2) would lose against col_kernel on short folds
+    T r = acc;
+    if (w == 0) {
+#pragma unroll
+        for (int i = 1; i < NW; ++i) r = Op::apply(r, lds[64 * i + lane]);
+    }
+    for (int n = per; n > 1;) {
+        const int h = (n + 1) / 2;
+        __syncthreads();
+        if (w == 0) lds[lane] = r;
+        __syncthreads();
+        if (w == 0 && sub + h < n) r = Op::apply(r, lds[lane + h * Q]);
+        n = h;
+    }
     if ((int)threadIdx.x >= Q) return;
-    T r = lds[threadIdx.x];
-    for (int i = 1; i < NW * per; ++i) r = Op::apply(r, lds[i / per * 64 + i % per * Q + threadIdx.x]);
     if (ksplit == 1) out[p * Q + threadIdx.x] = (S)r;
     else partials[(long long)blockIdx.x * 64 + threadIdx.x] = r;
 }

@@ -85,3 +85,18 @@ def test_short_folds_keep_four_partials(gpu, dtype, batches):
     a = np.random.default_rng(batches).normal(size=(batches, 517, 519)).astype(dtype)
     got = gpu.reduce(gpu.DeviceArray.from_numpy(a), "sum", 4).numpy(logical=True)
     assert np.array_equal(got[0], chain([strided(a, w, 4) for w in range(4)]))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows", [2, 3, 5, 8, 31, 32])
+@pytest.mark.parametrize("cols", [64, 100, 255])
+def test_few_kept_elements_fold_by_halves(gpu, dtype, rows, cols):
+    # more batches than blocks wanted, so that a fold is one block's
+    a = np.random.default_rng(cols + rows).normal(size=(2100, rows, cols)).astype(dtype)
+    got = gpu.reduce(gpu.DeviceArray.from_numpy(a), "sum", 2).numpy(logical=True)[:, :, 0]
+    x, per = np.moveaxis(a, 2, 0), 64 // rows
+    r = [chain([strided(x, w * per + s, 4 * per) for w in range(4)]) for s in range(per)]
+    while len(r) > 1:
+        h = (len(r) + 1) // 2
+        r = [r[i] + r[i + h] if i + h < len(r) else r[i] for i in range(h)]
+    assert np.array_equal(got, r[0])
