@@ -64,7 +64,6 @@ bool rx_column_wins(const CwProgram& P, const RxShape& SH)
     };
     int kept = 0, reduced = 0;
     for (int l = 0; l < P.nleaves; ++l) {
-        if (P.leaves[l].kind != CM_LEAF_STRIDED) return false;
         long long s[3];
         strides_of(P.leaves[l], s);
         bool vk = false, vr = false;
@@ -301,6 +300,10 @@ int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const 
     // also many short segments, whatever their layout: a block per segment
     // costs 0.8 ns a segment with hardly a thread at work
     const bool many_short = SH.L <= SHORT_FOLD && SH.nseg >= MANY_SEGMENTS;
+    // before the signature is looked up: a vector as a diagonal has the strides
+    // of the same vector broadcast over the columns
+    for (int l = 0; l < P.nleaves; ++l)
+        if (P.leaves[l].kind != CM_LEAF_STRIDED) return RX_JIT_DECLINED;
     if (!many_short && !rx_column_wins(P, SH)) return RX_JIT_DECLINED;
     const int units = units_for(chunk < SH.L ? chunk : SH.L);
     if ((SH.nseg + 63) / 64 * nchunk * units < MIN_WAVES) return RX_JIT_DECLINED;
@@ -324,6 +327,7 @@ int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const 
     for (int l = 0; l < P.nleaves; ++l) {
         const cm_leaf& L = P.leaves[l];
         jit::sig_add(sig, L.dtype);
+        jit::sig_add(sig, L.kind);
         jit::sig_add(sig, L.sr);
         jit::sig_add(sig, L.sc);
         jit::sig_add(sig, L.sb);

@@ -124,3 +124,19 @@ def test_bool_result(gpu):
     for op, ref in (("all", np.all), ("any", np.any)):
         got = both(cm, lambda: cm.reduce(A.expr() > cm.as_expr(np.float32(-2.5)), op, cm.capi.AXIS_COL).numpy(logical=True))
         assert np.array_equal(got, ref(a > -2.5, axis=2, keepdims=True))
+
+
+@pytest.mark.parametrize("diagonal_first", [False, True])
+def test_diagonal_leaf_after_its_broadcast_twin(gpu, diagonal_first):
+    """v.asDiagonal() has the strides of v broadcast over the columns: neither
+    may run the kernel generated for the other."""
+    cm = gpu
+    n, batches = 64, 512 + diagonal_first  # 32768 and more short folds; a shape of its own for each order
+    a, v = data((batches, n, n), np.float32, 9), data((1, n, 1), np.float32, 10)
+    A, V = cm.DeviceArray.from_numpy(a), cm.DeviceArray.from_numpy(v)
+    exact = a.astype(np.float64) * v
+    cases = [(V.expr(), exact), (V.expr().asDiagonal(), exact * np.eye(n))]
+    for leaf, x in reversed(cases) if diagonal_first else cases:
+        got = cm.reduce(A.expr() * leaf, "sum", cm.capi.AXIS_COL).numpy(logical=True)
+        bound = 2.0 ** -23 * (n + 4) * np.abs(x).sum(axis=2, keepdims=True)
+        assert np.all(np.abs(got - x.sum(axis=2, keepdims=True)) <= bound)
