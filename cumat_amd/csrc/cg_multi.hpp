@@ -1375,7 +1375,7 @@ static int cg_dia_prepare(cm_ctx_t ctx, Temps& tmp, int n, int nnz, int nb, cons
     void* buf = nullptr;
     const size_t plan_bytes = 256;
     static_assert(sizeof(DiaPlan) <= 256, "plan block");
-    if (tmp.get(plan_bytes + sizeof(VT) * (size_t)cap * nb, &buf) != CM_OK) return CM_OK;
+    if (tmp.get(plan_bytes + sizeof(VT) * (size_t)cap * nb, &buf, true) != CM_OK) return CM_OK;
     DiaPlan* plan = (DiaPlan*)buf;
     DiaPlan* host = (DiaPlan*)((char*)pinned_dev + CM_PINNED_BYTES / 2);
     *dia = (VT*)((char*)buf + plan_bytes);

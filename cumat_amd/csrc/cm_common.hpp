@@ -98,8 +98,10 @@ int scratch(cm_ctx_t ctx, int slot, size_t bytes, void** out);
 // while they run (coherent: device stores reach it without a cache flush).
 constexpr size_t CM_PINNED_BYTES = 4096;
 int pinned(cm_ctx_t ctx, void** host, void** dev);
-// Caching device allocator (the same pool as cm_malloc / cm_free).
-int dalloc(cm_ctx_t ctx, size_t bytes, void** out);
+// Caching device allocator (the same pool as cm_malloc / cm_free). optional:
+// CM_E_NOMEM without an error message where neither the cache nor the device
+// has the memory, and the cached blocks stay.
+int dalloc(cm_ctx_t ctx, size_t bytes, void** out, bool optional = false);
 // Stream-ordered on ctx's stream; ctx == nullptr: no queued work uses p.
 int dfree(cm_ctx_t ctx, void* p);
 // Drops the captured batched-CG graphs of a context (before it is destroyed).
@@ -120,9 +122,9 @@ struct Temps {
     // the blocks then return to the cache without a recorded event
     bool drained = false;
     explicit Temps(cm_ctx_t c) : ctx(c) {}
-    int get(size_t bytes, void** out)
+    int get(size_t bytes, void** out, bool optional = false)
     {
-        int s = dalloc(ctx, bytes, out);
+        int s = dalloc(ctx, bytes, out, optional);
         if (s == CM_OK) ptrs.push_back(*out);
         return s;
     }

@@ -113,7 +113,10 @@ static void* take_cached(int device, size_t cls, hipStream_t stream)
     return p;
 }
 
-static int device_alloc(int device, size_t bytes, hipStream_t stream, void** out)
+// optional: the caller does without the block where memory is short, so the
+// cached blocks stay and no error is reported. A failed hipMalloc's error is
+// taken out of HIP's last-error slot: the next launch check would report it.
+static int device_alloc(int device, size_t bytes, hipStream_t stream, void** out, bool optional = false)
 {
     size_t cls = size_class(bytes);
     {
@@ -127,6 +130,10 @@ static int device_alloc(int device, size_t bytes, hipStream_t stream, void** out
     }
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, cls);
+    if (e != hipSuccess && optional) {
+        (void)hipGetLastError();
+        return CM_E_NOMEM;
+    }
     if (e != hipSuccess) {
         // release the cache of this device and retry once (hipFree waits for
         // the device, so pending work on the cached blocks has finished)
@@ -142,7 +149,10 @@ static int device_alloc(int device, size_t bytes, hipStream_t stream, void** out
         }
         (void)hipGetLastError();
         e = hipMalloc(&p, cls);
-        if (e != hipSuccess) return fail(CM_E_NOMEM, "hipMalloc(%zu) failed: %s", cls, hipGetErrorString(e));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(CM_E_NOMEM, "hipMalloc(%zu) failed: %s", cls, hipGetErrorString(e));
+        }
     }
     count(CM_CNT_DEVICE_MEM_ALLOC);
     std::lock_guard<std::mutex> lk(g_alloc_mutex);
@@ -269,7 +279,10 @@ int scratch(cm_ctx_t ctx, int slot, size_t bytes, void** out)
     return CM_OK;
 }
 
-int dalloc(cm_ctx_t ctx, size_t bytes, void** out) { return device_alloc(ctx->device, bytes, ctx->stream, out); }
+int dalloc(cm_ctx_t ctx, size_t bytes, void** out, bool optional)
+{
+    return device_alloc(ctx->device, bytes, ctx->stream, out, optional);
+}
 int dfree(cm_ctx_t ctx, void* p) { return device_free(p, ctx ? ctx->stream : nullptr, ctx != nullptr); }
 
 int pinned(cm_ctx_t ctx, void** host, void** dev)

@@ -5,11 +5,28 @@
 // and from residuals evaluated on the host in double precision.
 #include <cuMat/IterativeLinearSolvers>
 
+#include <dlfcn.h>
+
 #include <random>
 
 #include "harness.h"
 
 using namespace cuMat;
+
+// The library's device allocations go through this definition, so that a test
+// can have the large ones refused. The refusal is the runtime's own (a size no
+// device has): it leaves what a full device leaves.
+static size_t g_refuse_from = ~(size_t)0;
+static int g_allocs = 0, g_refused = 0;
+extern "C" int hipMalloc(void** p, size_t bytes)
+{
+    typedef int (*Fn)(void**, size_t);
+    static const Fn real = (Fn)dlsym(RTLD_NEXT, "hipMalloc");
+    ++g_allocs;
+    if (bytes < g_refuse_from) return real(p, bytes);
+    ++g_refused;
+    return real(p, (size_t)1 << 60);
+}
 
 struct HostCsr {
     int n = 0;
@@ -380,6 +397,48 @@ TEST_CASE("dense A * x: row-major and column-major against the host, += and -=")
         for (int r = 0; r < rows; ++r) e += h[r + (size_t)rows * c];
         REQUIRE(h4[c] == e);
     }
+}
+
+TEST_CASE("Conjugate Gradient - no memory for the layout by diagonals")
+{
+    // 512^2: the work block takes 5 MB, the layout 7 MB
+    HostCsr h = poisson(512);
+    auto A = toDevice<float>(h);
+    auto bh = randomVector<float>(h.n, 7);
+    VectorXf b = VectorXf::fromHost(bh), x;
+    ConjugateGradient<SMatrixXf> cg(A);
+    cg.setTolerance(1e-5f).setPath(CM_CG_MULTIKERNEL);
+    cg.setMaxIterations(20);
+    x = cg.solve(b);  // too short for the layout: the work block comes into the cache
+    cg.setMaxIterations(5000);
+    g_refuse_from = (size_t)6 << 20;
+    try {
+        x = cg.solve(b);
+    } catch (...) {
+        g_refuse_from = ~(size_t)0;
+        throw;
+    }
+    g_refuse_from = ~(size_t)0;
+    REQUIRE(g_refused > 0);
+    REQUIRE(cg.error() <= 1e-5f);
+    REQUIRE(relResidual<float>(h, bh, x.toHostRowMajor()) <= 1e-3);
+    // the cached blocks are still there: only the layout itself is allocated now
+    g_allocs = 0;
+    x = cg.solve(b);
+    REQUIRE_MSG(g_allocs <= 1, g_allocs << " allocations");
+    REQUIRE(relResidual<float>(h, bh, x.toHostRowMajor()) <= 1e-3);
+}
+
+TEST_CASE("an allocation that fails leaves nothing for later calls to report")
+{
+    VectorXf v = VectorXf::Constant(1000, 2.0f);
+    g_refuse_from = (size_t)64 << 20;
+    void* p = nullptr;
+    const int status = cm_malloc(nullptr, (size_t)100 << 20, &p);
+    g_refuse_from = ~(size_t)0;
+    REQUIRE(status == CM_E_NOMEM);
+    VectorXf w = v + v;
+    REQUIRE(w.squaredNorm().getScalar() == 16000.0f);
 }
 
 HARNESS_MAIN()
