@@ -10,20 +10,27 @@
 // p[i + off[d]], a lane takes consecutive rows, and both the values and p
 // are read with contiguous wide loads and no LDS.
 //
-// The solve lays the matrix out itself, on its own stream and without
-// waiting: after its first CG_CHUNK iterations (a solve that stops there
-// pays nothing) cg_dia_detect_kernel collects the distinct offsets of a
-// sample of rows and cg_dia_convert_kernel writes the diagonals, checking
-// every stored entry. From iteration CG_DIA_FROM on K1 uses the diagonals if
-// every entry fitted; the iteration of the switch is fixed, so a solve gives
-// the same bits every time. A row's products are added in ascending column
+// The solve lays the matrix out itself, on its own stream, once it is known
+// to run for long enough: after every chunk of CG_CHUNK iterations from the
+// second on, the last two residuals that the host has heard of tell how many more a solve at that rate needs (cg_dia_pays). Then
+// cg_dia_detect_kernel collects the distinct offsets of a sample of rows and
+// cg_dia_convert_kernel writes the diagonals, checking every stored entry. A
+// chunk later, which is queued meanwhile, K1 uses the diagonals if every entry
+// fitted. The residuals decide, not the clock, so a solve switches at the same
+// iteration and gives the same bits every time. A row's products are added in ascending column
 // order, as the CSR product adds them (with fused multiply-adds); slots that
 // a row does not store hold 0 (their p is read inside the batch's own
 // vector, so a batch never meets another's values).
 //
-// Detection and conversion of 160^3 take 17 + 108 us, 4 iterations' gain.
+// Detection and conversion take 28 + 110 us at 160^3 (the gain of 4 iterations),
+// 17 + 6 at 512^2, 9 + 4 at 128^2; the detection of a matrix without diagonals
+// 15. Queued after the first chunk of every solve they made short ones slower:
+// 160^3 with 8 iterations 915 -> 1060 us, with 22 2140 -> 2290; now 915 and 2140
+// (58 iterations: 5350 without the layout, 4190 with it from iteration 24 on,
+// 4540 now, since the residuals of the first 24 foretell an earlier end).
 #pragma once
 #include <climits>
+#include <cmath>
 
 #include "cm_common.hpp"
 #include "spmv_core.hpp"
@@ -39,7 +46,23 @@ constexpr long long CG_DIA_MIN = 2048;
 constexpr int CG_DIA_SAMPLE = 2048;  // rows the detection looks at
 constexpr int CG_DIA_DETECT_BS = 1024;
 constexpr int CG_DIA_BS = 256;
-constexpr int CG_DIA_FROM = 3 * CG_CHUNK;  // first iteration over the diagonals
+// Iterations that have to be left, counted from the last residual that the host
+// has heard of, for the layout to pay: 16 of them pass before it is in use, and
+// the layout costs the gain of 4 (160^3) to about 40 (512^2, 13.8 and 13.3 us an
+// iteration). From CG_DIA_LARGE unknowns on the bytes bind. A residual falls ever
+// more slowly at first, so the prediction is short rather than long: at 160^3 a
+// solve of 58 iterations counts as 17 more after 16.
+constexpr int CG_DIA_PAYS = 64, CG_DIA_PAYS_LARGE = 16;
+constexpr long long CG_DIA_LARGE = 1 << 19;
+
+// Whether a solve that came from distance a to distance b (largest |r|^2 over
+// the threshold) in one chunk needs 'pays' more iterations from b on at that
+// rate. A residual that does not fall, and a tolerance of zero, mean yes.
+inline bool cg_dia_pays(float a, float b, int pays)
+{
+    if (!(b < a)) return true;
+    return !(CG_CHUNK * std::log((double)b) < pays * std::log((double)a / (double)b));
+}
 
 // What the detection found; written by the device into host-mapped memory
 // (so that the host reads it without a copy) and into device memory (for
@@ -47,15 +70,24 @@ constexpr int CG_DIA_FROM = 3 * CG_CHUNK;  // first iteration over the diagonals
 struct DiaPlan {
     int count;  // distinct offsets, ascending in off; 0: more than CG_DIA_MAX, or too sparse
     int bad;    // the conversion met an entry outside the diagonals
+    int ready;  // the conversion has ended (in the host's copy)
     int off[CG_DIA_MAX];
 };
 
+// The diagonals the two-launch form is built for (a row's operands stay in
+// registers).
+__host__ __device__ inline bool cg_dia_iter_takes(int count) { return count == 3 || count == 5 || count == 7; }
+
 // One block: the distinct column - row offsets of at most CG_DIA_SAMPLE rows
 // spread over the matrix, sorted. cap: elements of one batch's diagonals the
-// conversion may write (rows padded to ld).
+// conversion may write (rows padded to ld). Rows are far apart, so their pages
+// cost most of the time. The loops stay rolled: the code runs
+// once, and unrolled loads of eight entries, whose instructions have to be
+// fetched too, took 24 and 40 us at 512^2 and 160^3.
 static __global__ __launch_bounds__(CG_DIA_DETECT_BS) void cg_dia_detect_kernel(int n, const int* __restrict__ JA,
                                                                          const int* __restrict__ IA, long long ld,
-                                                                         long long cap, DiaPlan* __restrict__ plan,
+                                                                         long long cap, int fused,
+                                                                         DiaPlan* __restrict__ plan,
                                                                          DiaPlan* __restrict__ host)
 {
     __shared__ int tab[CG_DIA_MAX];
@@ -79,22 +111,22 @@ static __global__ __launch_bounds__(CG_DIA_DETECT_BS) void cg_dia_detect_kernel(
                 int cur = *(volatile int*)&tab[t];
                 if (cur == INT_MIN) cur = atomicCAS(&tab[t], INT_MIN, o);
                 if (cur == o || cur == INT_MIN) break;
+                if (t == 8 && *(volatile int*)&over) break;
             }
             if (t == CG_DIA_MAX) over = 1;
         }
     }
     __syncthreads();
+    if (tid >= 64) return;
+    const int v = tid < CG_DIA_MAX ? tab[tid] : INT_MIN;
+    int cnt = __popcll(__ballot(v != INT_MIN));
+    if (over || cnt * ld > cap || (fused && !cg_dia_iter_takes(cnt))) cnt = 0;
+    if (cnt && v != INT_MIN) {
+        int rank = 0;
+        for (int a = 0; a < CG_DIA_MAX; ++a) rank += tab[a] != INT_MIN && tab[a] < v;
+        plan->off[rank] = host->off[rank] = v;
+    }
     if (tid == 0) {
-        int cnt = 0;
-        while (cnt < CG_DIA_MAX && tab[cnt] != INT_MIN) ++cnt;
-        for (int a = 1; a < cnt; ++a) {
-            const int v = tab[a];
-            int j = a - 1;
-            for (; j >= 0 && tab[j] > v; --j) tab[j + 1] = tab[j];
-            tab[j + 1] = v;
-        }
-        if (over || cnt * ld > cap) cnt = 0;
-        for (int a = 0; a < cnt; ++a) plan->off[a] = host->off[a] = tab[a];
         plan->bad = host->bad = 0;
         plan->count = host->count = cnt;
     }
@@ -129,6 +161,9 @@ __global__ __launch_bounds__(CG_DIA_BS) void cg_dia_convert_kernel(int n, const 
     }
     if (k != e) host->bad = 1;
 }
+
+// Behind the conversion in the stream.
+static __global__ void cg_dia_ready_kernel(DiaPlan* __restrict__ host) { host->ready = 1; }
 
 // Arguments of the product: everything that does not change between
 // iterations.

@@ -2,8 +2,8 @@
 // right-hand sides), fence-free.
 //
 // Per iteration i, three launches (the default form):
-//   K1  tmp = A p, per-block partial p.tmp (from iteration CG_DIA_FROM on over
-//       the matrix's diagonals where it has few, cg_dia.hpp)
+//   K1  tmp = A p, per-block partial p.tmp (over the matrix's
+//       diagonals where it has few and the solve is long, cg_dia.hpp)
 //   K2  every block reduces K1's partials of its batch in the same fixed
 //       order -> the same alpha = absNew[i&1] / p.tmp; r -= alpha tmp
 //       (and x += alpha p for small systems); per-block partials of |r|^2
@@ -117,7 +117,22 @@ struct CgMirror {
     int biters[CG_MAXB];
     double berr[CG_MAXB];
     int xset[CG_MAXB];  // batch's x holds a value (guess, zeros or an update)
+    // how far the solve was from its end before the first iteration and after
+    // each chunk, a ring of four: one word of (iterations + 1) << 32 and the
+    // bits of a float (cg_publish_distance)
+    unsigned long long distance[4];
 };
+
+// The largest |r|^2 / threshold of the running batches after 'done' iterations,
+// a multiple of CG_CHUNK. Called by the first wavefront of block (0, 0), lane k
+// with batch k's values; the host predicts the solve's end from it.
+template <typename T>
+__device__ __forceinline__ void cg_publish_distance(CgMirror* mirror, int done, bool running, T rr, T thr)
+{
+    const float f = wave_reduce<OpMax>(running ? (float)(rr / thr) : 0.f);
+    if (threadIdx.x == 0)
+        mirror->distance[(done / CG_CHUNK) & 3] = ((unsigned long long)(done + 1) << 32) | __float_as_uint(f);
+}
 
 // Sum of G partials (stride 'stride' between consecutive ones) in a fixed
 // order; identical in every block. lds: BS/64 entries.
@@ -478,6 +493,11 @@ __global__ __launch_bounds__(CG_BS) void cg_setup_finalize_kernel(int G, int B, 
             if (threadIdx.x == 0) tot[c][k] = v;
         }
     __syncthreads();
+    if (threadIdx.x < 64) {
+        const int k = threadIdx.x;
+        const T rhs = k < B ? tot[0][k] : T(1);
+        cg_publish_distance(mirror, 0, k < B && !(rhs < tol * tol), k < B ? tot[1][k] : T(0), tol * tol * rhs);
+    }
     if (threadIdx.x == 0) {
         bool all_zero = true, all_conv = true, all_done = true;
         T m = 0;
@@ -743,6 +763,9 @@ __global__ __launch_bounds__(CG_BS) void cg_iter_kernel(int n, int it, int B, in
         const bool own_prev = per_batch && st->bdone[bb] != CG_RUNNING;
         const bool own_conv = own_prev || rr_s[bb] < st->thr[bb];
         const T absOld = st->absNew[prev & 1][bb];
+        if (blockIdx.x == 0 && bb == 0 && threadIdx.x < 64 && (prev % CG_CHUNK) == CG_CHUNK - 1)
+            cg_publish_distance(mirror, it, lane < B && !(per_batch && st->bdone[lane] != CG_RUNNING),
+                                lane < B ? rr_s[lane] : T(0), lane < B ? st->thr[lane] : T(1));
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             if (per_batch && !own_prev) {
                 st->berr[bb] = sqrt((double)(rr_s[bb] / st->rhs2[bb]));
@@ -1158,6 +1181,8 @@ __global__ __launch_bounds__(CG_BS) void cg_pupdate_kernel(int n, int it_arg, in
     // this batch's last iteration: converged, or the iteration limit
     const bool last = (per_batch ? own_conv : all) || it + 1 >= max_iter;
     const bool publish = last || (it % CG_CHUNK) == CG_CHUNK - 1 || (per_batch && own_conv);
+    if (blockIdx.x == 0 && bb == 0 && threadIdx.x < 64 && (it % CG_CHUNK) == CG_CHUNK - 1)
+        cg_publish_distance(mirror, it + 1, !prev_k, lane < B ? rr_s[lane] : T(0), lane < B ? thr_s[lane] : T(1));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (per_batch && !own_prev) {
             const double e = sqrt((double)(rr_s[bb] / rhs_s[bb]));
@@ -1347,10 +1372,6 @@ struct CgBatchOpts {
     const BlockOp* block = nullptr;  // a block-CSR operator replaces the CSR matrix (FP32)
 };
 
-// The diagonals the two-launch form is built for (a row's operands stay in
-// registers).
-inline bool cg_dia_iter_takes(int count) { return count == 3 || count == 5 || count == 7; }
-
 template <typename VT, typename T>
 static void launch_cg_dia_iter(hipStream_t stream, int n, int it, int B, int G1, int G2, const DiaArgs& A,
                                const VT* dia, const T* invd, int istride, const T* r, const T* pprev, T* pnext, T* tmp,
@@ -1368,7 +1389,7 @@ static void launch_cg_dia_iter(hipStream_t stream, int n, int it, int B, int G1,
 // Queues the layout by diagonals; *dia stays NULL where it does not pay or
 // no memory is left (the solve then keeps the CSR product).
 template <typename VT>
-static int cg_dia_prepare(cm_ctx_t ctx, Temps& tmp, int n, int nnz, int nb, const int* JA, const int* IA,
+static int cg_dia_prepare(cm_ctx_t ctx, Temps& tmp, bool fused, int n, int nnz, int nb, const int* JA, const int* IA,
                           const VT* vals, long long vstride, long long ld, void* pinned_dev, VT** dia)
 {
     const long long cap = (long long)nnz + nnz / 4 + 8 * 32;
@@ -1379,11 +1400,14 @@ static int cg_dia_prepare(cm_ctx_t ctx, Temps& tmp, int n, int nnz, int nb, cons
     DiaPlan* plan = (DiaPlan*)buf;
     DiaPlan* host = (DiaPlan*)((char*)pinned_dev + CM_PINNED_BYTES / 2);
     *dia = (VT*)((char*)buf + plan_bytes);
-    cg_dia_detect_kernel<<<1, CG_DIA_DETECT_BS, 0, ctx->stream>>>(n, JA, IA, ld, cap, plan, host);
+    cg_dia_detect_kernel<<<1, CG_DIA_DETECT_BS, 0, ctx->stream>>>(n, JA, IA, ld, cap, fused ? 1 : 0, plan, host);
     CM_LAUNCH_CHECK();
     cg_dia_convert_kernel<VT><<<dim3(div_up(ld, CG_DIA_BS), nb), CG_DIA_BS, 0, ctx->stream>>>(
         n, JA, IA, vals, vstride, ld, *dia, plan, host);
     CM_LAUNCH_CHECK();
+    cg_dia_ready_kernel<<<1, 1, 0, ctx->stream>>>(host);
+    CM_LAUNCH_CHECK();
+    count(CM_CNT_CG_LAYOUT);
     return CM_OK;
 }
 
@@ -1473,6 +1497,8 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     // the previous solve on this context left its final state here
     hm->status = CG_RUNNING;
     hm->it_done = -1;
+    for (int k = 0; k < 4; ++k) hm->distance[k] = 0;
+    hplan->ready = 0;
     int launches = 0;
     auto t0 = std::chrono::steady_clock::now();
     int Gs = G1;
@@ -1521,37 +1547,50 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     // until the mirror shows the chunk before the last one tested (kernels
     // publish every CG_CHUNK-th iteration), and stop once the solve ended.
     // If the stream drains first, every launched iteration has run.
-    auto wait_mirror = [&](int need) {
+    auto wait_for = [&](auto arrived) {
         count(CM_CNT_HOST_SYNC);
         for (unsigned k = 1;; ++k) {
-            if (hm->status != CG_RUNNING || hm->it_done >= need) return;
+            if (hm->status != CG_RUNNING || arrived()) return;
             if ((k & 255) == 0 && hipStreamQuery(ctx->stream) == hipSuccess) return;
             __builtin_ia32_pause();
         }
     };
     int it = 0;
-    // K1 over the diagonals (cg_dia.hpp): laid out after the first chunk if
-    // enough iterations are left to pay for it, used from CG_DIA_FROM on
-    const bool try_dia = !dense && !block && (fused || N >= CG_DIA_MIN) && max_iter >= CG_DIA_FROM + 2 * CG_CHUNK && nnz > 0;
+    // K1 over the diagonals (cg_dia.hpp): laid out once the solve is known to
+    // need enough iterations to pay for it, used a chunk later
+    bool try_dia = !dense && !block && (fused || N >= CG_DIA_MIN) && nnz > 0;
+    const int dia_pays = N >= CG_DIA_LARGE ? CG_DIA_PAYS_LARGE : CG_DIA_PAYS;
+    // the distance after so many iterations, once it has arrived
+    auto distance = [&](int done) {
+        volatile unsigned long long* word = &hm->distance[(done / CG_CHUNK) & 3];
+        wait_for([&] { return (int)(*word >> 32) == done + 1; });
+        const unsigned bits = (unsigned)*word;
+        float f;
+        memcpy(&f, &bits, 4);
+        return f;
+    };
+    int dia_from = -1;
     const long long dia_ld = ((long long)n + 7) / 8 * 8;
     DiaArgs da{};
     VT* dia = nullptr;
     const DiaArgs* dia_on = nullptr;
     while (it < max_iter) {
         int todo = std::min(CG_CHUNK, max_iter - it);
-        if (try_dia && it == CG_CHUNK)
-            CM_TRY((cg_dia_prepare<VT>(ctx, tmp, n, nnz, nbi, JA, IA, vals, vstride, dia_ld, mirror_dev, &dia)));
-        if (dia && !dia_on && it == CG_DIA_FROM && hplan->count > 0 && !hplan->bad) {
-            // the host has waited for an iteration queued behind the conversion
+        // (the last chunk is still running: the two before it are known)
+        if (try_dia && it >= 2 * CG_CHUNK && max_iter - it >= dia_pays &&
+            cg_dia_pays(distance(it - 2 * CG_CHUNK), distance(it - CG_CHUNK), dia_pays) && hm->status == CG_RUNNING) {
+            CM_TRY((cg_dia_prepare<VT>(ctx, tmp, fused, n, nnz, nbi, JA, IA, vals, vstride, dia_ld, mirror_dev, &dia)));
+            try_dia = false;
+            dia_from = it + CG_CHUNK;
+        }
+        if (dia && it == dia_from) wait_for([&] { return hplan->ready != 0; });
+        if (dia && it == dia_from && hplan->ready && hplan->count > 0 && !hplan->bad) {
             da.count = hplan->count;
             da.ld = dia_ld;
             da.bstride = vstride ? da.count * dia_ld : 0;
             for (int d = 0; d < da.count; ++d) da.off[d] = hplan->off[d];
-            if (fused && !cg_dia_iter_takes(da.count)) {
-                dia = nullptr;
-                continue;
-            }
             dia_on = &da;
+            count(CM_CNT_CG_DIAGONALS);
             if (!fused) G1 = walk_grid(div_up(n, cg_dia_rows_per_block(n)), gcap);
         }
         for (int k = 0; k < todo; ++k, ++it) {
@@ -1582,7 +1621,7 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
         CM_LAUNCH_CHECK();
         launches += (fused ? 2 : 3) * todo;
         if (it > CG_CHUNK && it < max_iter) {
-            wait_mirror(it - CG_CHUNK - 1);
+            wait_for([&] { return hm->it_done >= it - CG_CHUNK - 1; });
             if (hm->status != CG_RUNNING) break;
         }
     }

@@ -75,7 +75,9 @@ public:
         // kernels compiled / launched for component-wise programs at run time
         HostSync = CM_CNT_HOST_SYNC,
         JitCompile = CM_CNT_JIT_COMPILE,
-        JitLaunch = CM_CNT_JIT_LAUNCH
+        JitLaunch = CM_CNT_JIT_LAUNCH,
+        CgLayout = CM_CNT_CG_LAYOUT,
+        CgDiagonals = CM_CNT_CG_DIAGONALS
     };
     static Profiling& instance()
     {

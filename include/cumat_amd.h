@@ -96,7 +96,11 @@ enum cm_counter {
      * component-wise program, and launches of such kernels (cm_jit_mode) */
     CM_CNT_JIT_COMPILE = 10,
     CM_CNT_JIT_LAUNCH = 11,
-    CM_CNT_COUNT = 12
+    /* no reference counterpart: CG solves that laid their matrix out by
+     * diagonals, and those whose iterations then ran over that layout */
+    CM_CNT_CG_LAYOUT = 12,
+    CM_CNT_CG_DIAGONALS = 13,
+    CM_CNT_COUNT = 14
 };
 
 typedef struct cm_context* cm_ctx_t;

@@ -2,8 +2,7 @@
 forms it takes (tile edges, missing entries, several right-hand sides, values
 per batch, FP64) and those it must leave to the CSR product (too many
 diagonals, columns out of order, an entry that the sample did not show),
-against the CPU oracle. Every system needs more iterations than the solve
-runs before it switches (24)."""
+against the CPU oracle; and which solves lay their matrix out at all."""
 import numpy as np
 import pytest
 
@@ -116,3 +115,41 @@ def test_values_per_batch(gpu, orc, batches):
                             max_iter=5000)
         assert abs(its[k] - it) <= 2
         np.testing.assert_allclose(x[k].cpu().numpy(), xo, rtol=0, atol=1e-8 * np.abs(xo).max())
+
+
+def poisson_solver(cm, side, path):
+    from cumat_amd.problems import poisson2d
+    n = side * side
+    JA, IA, V = poisson2d(side)
+    b = cm.DeviceArray.from_numpy(np.random.default_rng(side).uniform(-1, 1, n).astype(np.float32))
+    return cm.ConjugateGradient(cm.SparseMatrix.from_csr(n, n, JA, IA, V), path=path), b
+
+
+def layouts(cm, cg, b, tol, max_iter=2000):
+    """(iterations, layouts queued, solves over the diagonals)"""
+    cm.reset_counters()
+    cg.setTolerance(tol).setMaxIterations(max_iter).solve(b)
+    c = cm.counters()
+    return cg.iterations(), c["CgLayout"], c["CgDiagonals"]
+
+
+@pytest.mark.parametrize("path,side", [(1, 128), (1, 600), (3, 128)])
+def test_short_solves_lay_nothing_out(gpu, path, side):
+    """Below about 30 iterations the layout costs more than it gains."""
+    cm = gpu
+    cg, b = poisson_solver(cm, side, path)
+    seen = [layouts(cm, cg, b, tol) for tol in (0.5, 0.3, 0.2, 0.14, 0.1, 0.07, 0.05)]
+    assert min(it for it, _, _ in seen) <= 8 and max(it for it, _, _ in seen) >= 20
+    for it, queued, used in seen:
+        if it <= 32:
+            assert (queued, used) == (0, 0), it
+    assert layouts(cm, cg, b, 0.0, 50)[1:] == (0, 0)  # too few iterations allowed
+    it, queued, used = layouts(cm, cg, b, 1e-6)
+    assert it > 150 and (queued, used) == (1, 1)
+
+
+def test_the_switch_is_reproducible(gpu):
+    cm = gpu
+    cg, b = poisson_solver(cm, 300, 1)
+    runs = [cg.setTolerance(1e-6).setMaxIterations(2000).solve(b).numpy().tobytes() for _ in range(5)]
+    assert len(set(runs)) == 1
