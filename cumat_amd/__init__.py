@@ -37,7 +37,7 @@ def counters() -> dict:
     """Profiling counters (cuMat::Profiling, cuMat/src/Profiling.h:23-109)."""
     names = ["DeviceMemAlloc", "DeviceMemFree", "EvalAny", "EvalCwise", "EvalCwiseSparse",
              "EvalReduction", "EvalMatmulSparse", "KernelLaunch", "EvalMatmul", "HostSync",
-             "JitCompile", "JitLaunch", "CgLayout", "CgDiagonals"]
+             "JitCompile", "JitLaunch", "CgLayout", "CgDiagonals", "CgWalk"]
     out = {}
     for i, n in enumerate(names):
         v = C.c_longlong(0)

@@ -57,7 +57,11 @@ struct ResidentArgs {
     int* iters_out;       // per system
     T* err_out;           // per system
     unsigned* queue;      // queue[0]: work counter, queue[1]: invalid-pattern
-                          // flag (both zeroed before launch)
+                          // flag, queue[2]: systems listed in walk, queue[3]:
+                          // systems walked beside the register form (zeroed
+                          // before launch)
+    int* walk;            // the register form lists the systems here that it
+                          // leaves to the walking kernel
     int nnz_total;        // entries of IA / vals (every JA value must lie in
                           // [0, nnz_total])
 };
@@ -74,17 +78,25 @@ constexpr int resident_group(int rpt) { return rpt % 4 == 0 ? 4 : (rpt % 3 == 0 
 // wavefront are consecutive words, and a thread's reads on one diagonal are
 // one address plus constants. A slot the row does not store holds 0; its read
 // may leave the system by up to the largest offset, into RESIDENT_GUARD zeros
-// on either side of p. Systems with other patterns or longer offsets, and
-// W = 0, walk their CSR rows in memory each iteration.
+// on either side of p. Systems with other patterns or longer offsets walk
+// their CSR rows in memory each iteration; beyond four row slots they are listed
+// for a launch of W = 0, which only walks and keeps p in LDS alone.
 //
 // What bounds the walk is its chain of dependent, uncoalesced loads (8 bytes
-// per entry from L2, lanes 20 bytes apart); what bounds the register form is
-// the LDS reads (W + 1 per row) and the latency of the two reductions and
-// three barriers of an iteration. Measured on MI355X, us per iteration of
-// one system, walking / in registers: 5 diagonals FP32 1024 rows 2.9 / 1.3,
-// 4096 7.2 / 1.7, 9216 14.5 / 2.8; 7 diagonals 4096 2.1, 5832 2.7; FP64 5
-// diagonals 4096 2.3. 4096 systems of 16^2 to 96^2: 5.35 -> 1.87 ms.
+// per entry from L2, lanes 20 bytes apart), so it wants as many wavefronts as
+// fit: its own kernel, without the matrix's registers, 1024 threads for one
+// system of more than 2048 rows. What bounds the register form is the LDS reads
+// (W + 1 per row) and the latency of the two reductions and three barriers of an
+// iteration. Measured on MI355X, us per iteration of one system, walking / in
+// registers: 5 diagonals FP32 1024 rows 2.9 / 1.3, 4096 7.2 / 1.7, 9216 14.5 /
+// 2.6; 7 diagonals 4096 2.1, 5832 2.7; FP64 5 diagonals 4096 2.3. 4096 systems of
+// 16^2 to 96^2: 5.35 -> 1.65 ms. Walking in the register form's kernel and shape
+// instead: 2048 permuted systems of 64^2 4.3 -> 6.0 ms, of 16^2 to 96^2 4.3 -> 5.4,
+// one of 8100 rows 13.1 -> 14.8 us per iteration. Up to four row slots (74
+// registers) the walk stays there: it costs no occupancy, and a second launch
+// would cost more (2048 systems of 16^2 to 32^2 722 us, 878 with the launch).
 constexpr int RESIDENT_GUARD = 1024;
+constexpr bool resident_lists(int rpt, int w) { return w > 0 && rpt > 4; }
 template <typename T, int BS, int RPT, int W>
 constexpr size_t resident_lds(int nmax)
 {
@@ -99,12 +111,14 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
     constexpr int NW = BS / 64;
     constexpr int GR = resident_group(RPT);
     constexpr int WR = W ? W : 1;
+    constexpr bool LIST = resident_lists(RPT, W);  // systems that do not fit are left to W = 0
     __shared__ T red[2 * NW];
     __shared__ T red1[NW];
     __shared__ int s_sys;
     __shared__ int s_bad;
     __shared__ int s_off[WR + 1];  // the diagonals, ascending; INT_MIN: free
-    __shared__ int s_walk;         // the system does not fit the register form
+    __shared__ int s_walk;         // the system does not fit the register form: by the sample,
+    __shared__ int s_walk2;        // by its entries
     const int tid = threadIdx.x;
     // sum over the block with one barrier: the caller's next use of the same
     // buffer lies behind another barrier of the iteration
@@ -144,6 +158,7 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
             s_sys = (int)atomicAdd(A.queue, 1u);
             s_bad = 0;
             s_walk = W == 0;
+            s_walk2 = 0;
         }
         if (tid <= WR) s_off[tid] = INT_MIN;
         __syncthreads();
@@ -203,7 +218,9 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
         // system is not solved: iterations -1, error NaN, queue[1] set.
         // The same pass loads the entries of the register form.
         // (Row bounds first, then the entries of GR rows at a time: the loads
-        // of a group are in flight together.)
+        // of a group are in flight together.) A system that the sample has
+        // turned away loads nothing where it is left to another launch.
+        const bool load = !LIST || __builtin_amdgcn_readfirstlane(s_walk) == 0;
         bool bad = false, walk = false;
         T val[RPT][WR];
         int rs[RPT], re[RPT];
@@ -215,7 +232,7 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
 #pragma unroll
                 for (int k = 0; k < WR; ++k) val[g + u][k] = T(0);
             }
-            if (g * BS >= n) continue;
+            if (!load || g * BS >= n) continue;
 #pragma unroll
             for (int u = 0; u < GR; ++u) {
                 const int i = tid + (g + u) * BS;
@@ -227,7 +244,7 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
         }
 #pragma unroll
         for (int g = 0; g < RPT; g += GR) {
-            if (g * BS >= n) continue;
+            if (!load || g * BS >= n) continue;
             int c[GR][WR];
             T v[GR][WR];
 #pragma unroll
@@ -265,7 +282,7 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
                     walk |= hits != len;
                 } else {
                     walk = true;
-                    for (int k = rs[j]; k < re[j]; ++k) {
+                    for (int k = rs[j]; !LIST && k < re[j]; ++k) {
                         const int cc = A.IA[k] - row0;
                         bad |= (cc < 0) | (cc >= n);
                     }
@@ -275,7 +292,7 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
         // one flag for the workgroup, read into a scalar register so that the
         // branches on it are uniform
         if (bad) s_bad = 1;
-        if (walk) s_walk = 1;
+        if (walk) s_walk2 = 1;
         __syncthreads();
         // Every path ends at the barrier at the end of the loop body: the
         // loop has no early "continue". (With one, the compiled loop sent the
@@ -283,17 +300,31 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
         // while thread 0 waited to fetch the next system, so a workgroup that
         // met an invalid system spun on it for ever.)
         const bool invalid = __builtin_amdgcn_readfirstlane(s_bad) != 0;
-        const bool regs = W > 0 && __builtin_amdgcn_readfirstlane(s_walk) == 0;
+        const bool regs = W > 0 && __builtin_amdgcn_readfirstlane(s_walk | s_walk2) == 0;
         if (invalid && tid == 0) {
             if (A.iters_out) A.iters_out[sys] = -1;
             if (A.err_out) A.err_out[sys] = T(NAN);
             atomicOr(A.queue + 1, 1u);
         }
-        if (!invalid) {
-            T xr[RPT], rr[RPT], id[RPT], pr[RPT], tmp[RPT];
-            // tmp = A p (p in LDS); rows past n get 0
+        if (W > 0 && !invalid && !regs && tid == 0) {
+            if (LIST) A.walk[atomicAdd(A.queue + 2, 1u)] = sys;
+            else atomicAdd(A.queue + 3, 1u);
+        }
+        if (!invalid && (regs || !LIST)) {
+            T xr[RPT], rr[RPT], id[RPT], pr[W > 0 ? RPT : 1], tmp[RPT];
+            // (A p)[i] from the CSR row
+            auto walk_row = [&](int i) {
+                const int s = A.JA[row0 + i], e = A.JA[row0 + i + 1];
+                T acc = T(0);
+                if (s < e) {
+                    acc = A.vals[s] * pl[A.IA[s] - row0];
+                    for (int k = s + 1; k < e; ++k) acc += A.vals[k] * pl[A.IA[k] - row0];
+                }
+                return acc;
+            };
+            // W > 0: tmp = A p (p in LDS); rows past n get 0
             auto product = [&]() {
-                if (regs) {
+                if (LIST || regs) {
 #pragma unroll
                     for (int g = 0; g < RPT; g += GR) {
                         if (g * BS < n) {
@@ -318,15 +349,7 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
 #pragma unroll
                     for (int j = 0; j < RPT; ++j) {
                         const int i = tid + j * BS;
-                        T acc = T(0);
-                        if (i < n) {
-                            const int s = A.JA[row0 + i], e = A.JA[row0 + i + 1];
-                            if (s < e) {
-                                acc = A.vals[s] * pl[A.IA[s] - row0];
-                                for (int k = s + 1; k < e; ++k) acc += A.vals[k] * pl[A.IA[k] - row0];
-                            }
-                        }
-                        tmp[j] = acc;
+                        tmp[j] = i < n ? walk_row(i) : T(0);
                     }
                 }
             };
@@ -336,12 +359,12 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
                 int i = tid + j * BS;
                 xr[j] = T(0);
                 id[j] = T(1);
-                tmp[j] = T(0);
+                if constexpr (W > 0) tmp[j] = T(0);
                 if (i < n) {
                     if (A.invd) id[j] = A.invd[row0 + i];
                     else {
                         T d = T(0);
-                        if (regs) {
+                        if (LIST || regs) {
 #pragma unroll
                             for (int k = 0; k < WR; ++k)
                                 if (k < cnt && off[k] == 0) d = val[j][k];
@@ -356,10 +379,11 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
                 if (W > 0 || i < n) pl[i] = xr[j];  // the register form: zeros past n
             }
             __syncthreads();
-            if (A.use_guess) {
-                product();
-                __syncthreads();
-            }
+            if constexpr (W > 0)
+                if (A.use_guess) {
+                    product();
+                    __syncthreads();
+                }
             T bb = 0, r2 = 0;
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
@@ -367,7 +391,10 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
                 rr[j] = T(0);
                 if (i < n) {
                     T bv = A.b[row0 + i];
-                    rr[j] = bv - tmp[j];
+                    T ax = T(0);
+                    if constexpr (W > 0) ax = tmp[j];
+                    else if (A.use_guess) ax = walk_row(i);
+                    rr[j] = bv - ax;
                     bb += bv * bv;
                     r2 += rr[j] * rr[j];
                 }
@@ -391,11 +418,12 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
 #pragma unroll
                 for (int j = 0; j < RPT; ++j) {
                     int i = tid + j * BS;
-                    pr[j] = T(0);
+                    if constexpr (W > 0) pr[j] = T(0);
                     if (i < n) {
-                        pr[j] = id[j] * rr[j];
-                        pl[i] = pr[j];
-                        absNew += rr[j] * pr[j];
+                        const T pv = id[j] * rr[j];
+                        if constexpr (W > 0) pr[j] = pv;
+                        pl[i] = pv;
+                        absNew += rr[j] * pv;
                     }
                 }
                 absNew = sum1(absNew);  // also orders the LDS writes
@@ -404,19 +432,35 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
                 int it = 0;
                 // rows past n hold zeros throughout
                 while (it < A.max_iter) {
-                    product();
                     T pap = 0;
+                    if constexpr (W > 0) {
+                        product();
 #pragma unroll
-                    for (int j = 0; j < RPT; ++j) pap += pr[j] * tmp[j];
+                        for (int j = 0; j < RPT; ++j) pap += pr[j] * tmp[j];
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < RPT; ++j) {
+                            const int i = tid + j * BS;
+                            tmp[j] = T(0);
+                            if (i < n) {
+                                tmp[j] = walk_row(i);
+                                pap += pl[i] * tmp[j];
+                            }
+                        }
+                    }
                     pap = sum1(pap);
                     const T alpha = absNew / pap;
                     T sr = 0, sz = 0;
 #pragma unroll
                     for (int j = 0; j < RPT; ++j) {
-                        xr[j] += alpha * pr[j];
-                        rr[j] -= alpha * tmp[j];
-                        sr += rr[j] * rr[j];
-                        sz += rr[j] * (id[j] * rr[j]);
+                        const int i = tid + j * BS;
+                        if (W > 0 || i < n) {
+                            if constexpr (W > 0) xr[j] += alpha * pr[j];
+                            else xr[j] += alpha * pl[i];
+                            rr[j] -= alpha * tmp[j];
+                            sr += rr[j] * rr[j];
+                            sz += rr[j] * (id[j] * rr[j]);
+                        }
                     }
                     sum2(sr, sz);
                     rsq = sr;
@@ -426,8 +470,12 @@ __global__ __launch_bounds__(BS) void cg_resident_kernel(const ResidentArgs<T> A
 #pragma unroll
                     for (int j = 0; j < RPT; ++j) {
                         int i = tid + j * BS;
-                        pr[j] = id[j] * rr[j] + beta * pr[j];
-                        if (W > 0 ? j / GR * GR * BS < n : i < n) pl[i] = pr[j];
+                        if constexpr (W > 0) {
+                            pr[j] = id[j] * rr[j] + beta * pr[j];
+                            if (j / GR * GR * BS < n) pl[i] = pr[j];
+                        } else {
+                            if (i < n) pl[i] = id[j] * rr[j] + beta * pl[i];
+                        }
                     }
                     __syncthreads();
                     ++it;
@@ -505,27 +553,42 @@ static int launch_resident_w(cm_ctx_t ctx, const ResidentArgs<T>& A, int nmax, i
         CM_RES(32);
     }
 #undef CM_RES
-    if constexpr (W > 0) return launch_resident_w<T, BS, 0>(ctx, A, nmax, grid, gpc);
     return fail(CM_E_UNSUPPORTED, "resident CG: %d rows exceed %d threads x tile", nmax, BS);
 }
 
-// nnz_mean: stored entries per row, rounded up; the diagonals to expect
-template <typename T, int BS>
-static int launch_resident_bs(cm_ctx_t ctx, const ResidentArgs<T>& A, int nmax, int grid, int gpc, int nnz_mean)
+// Diagonals of the register form for systems of up to nmax rows and nnz_mean
+// stored entries per row (rounded up): 5, 7, or 0 where they have to walk.
+template <typename T>
+static int resident_diagonals(int bs, int nmax, int nnz_mean)
 {
-    if (nnz_mean <= 5) return launch_resident_w<T, BS, 5>(ctx, A, nmax, grid, gpc);
-    if (nnz_mean <= 7) return launch_resident_w<T, BS, 7>(ctx, A, nmax, grid, gpc);
+    if (nnz_mean > 7) return 0;
+    const int w = nnz_mean <= 5 ? 5 : 7;
+    int rpt = 0;
+    switch (bs) {
+    case 256: rpt = w == 5 ? resident_max_rpt<T, 256, 5>() : resident_max_rpt<T, 256, 7>(); break;
+    case 512: rpt = w == 5 ? resident_max_rpt<T, 512, 5>() : resident_max_rpt<T, 512, 7>(); break;
+    case 1024: rpt = w == 5 ? resident_max_rpt<T, 1024, 5>() : resident_max_rpt<T, 1024, 7>(); break;
+    default: break;
+    }
+    return nmax <= rpt * bs ? w : 0;
+}
+
+template <typename T, int BS>
+static int launch_resident_bs(cm_ctx_t ctx, const ResidentArgs<T>& A, int nmax, int grid, int gpc, int w)
+{
+    if (w == 5) return launch_resident_w<T, BS, 5>(ctx, A, nmax, grid, gpc);
+    if (w == 7) return launch_resident_w<T, BS, 7>(ctx, A, nmax, grid, gpc);
     return launch_resident_w<T, BS, 0>(ctx, A, nmax, grid, gpc);
 }
 
+// w: resident_diagonals, or 0 for the walking kernel
 template <typename T>
-static int launch_resident(cm_ctx_t ctx, const ResidentArgs<T>& A, int nmax, int bs, int grid, int nnz_mean,
-                           int gpc = 0)
+static int launch_resident(cm_ctx_t ctx, const ResidentArgs<T>& A, int nmax, int bs, int grid, int w, int gpc = 0)
 {
     switch (bs) {
-    case 256: return launch_resident_bs<T, 256>(ctx, A, nmax, grid, gpc, nnz_mean);
-    case 512: return launch_resident_bs<T, 512>(ctx, A, nmax, grid, gpc, nnz_mean);
-    case 1024: return launch_resident_bs<T, 1024>(ctx, A, nmax, grid, gpc, nnz_mean);
+    case 256: return launch_resident_bs<T, 256>(ctx, A, nmax, grid, gpc, w);
+    case 512: return launch_resident_bs<T, 512>(ctx, A, nmax, grid, gpc, w);
+    case 1024: return launch_resident_bs<T, 1024>(ctx, A, nmax, grid, gpc, w);
     default: return fail(CM_E_ARG, "resident CG: block size %d (256, 512 or 1024)", bs);
     }
 }
@@ -558,23 +621,34 @@ static int pcg_resident(cm_ctx_t ctx, int n, int nnz, const int* JA, const int* 
     A.iters_out = (int*)io;
     A.err_out = (T*)eo;
     A.queue = (unsigned*)q;
+    A.walk = (int*)((char*)q + 64);
     A.nnz_total = nnz;
     auto t0 = std::chrono::steady_clock::now();
-    CM_TRY(launch_resident<T>(ctx, A, n, n <= 9216 ? 512 : 1024, 1, (int)div_up(nnz, n)));
     int hi = 0;
     T he = 0;
-    unsigned bad = 0;
-    CM_HIP(hipMemcpyAsync(&hi, io, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    CM_HIP(hipMemcpyAsync(&he, eo, sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
-    CM_HIP(hipMemcpyAsync(&bad, (unsigned*)q + 1, sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
-    CM_TRY(::cm::host_sync(ctx));
-    CM_REQUIRE(!bad, CM_E_ARG, "resident CG: a row pointer or column index lies outside the %d x %d matrix", n, n);
+    unsigned flags[3] = {0, 0, 0};  // invalid pattern, left to the walking kernel, walked
+    auto run = [&](int bs, int w) {
+        CM_TRY(launch_resident<T>(ctx, A, n, bs, 1, w));
+        CM_HIP(hipMemcpyAsync(&hi, io, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        CM_HIP(hipMemcpyAsync(&he, eo, sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
+        CM_HIP(hipMemcpyAsync(flags, A.queue + 1, sizeof(flags), hipMemcpyDeviceToHost, ctx->stream));
+        return ::cm::host_sync(ctx);
+    };
+    const int bs = n <= 9216 ? 512 : 1024, w = resident_diagonals<T>(bs, n, (int)div_up(nnz, n));
+    if (w) CM_TRY(run(bs, w));
+    const bool walk = !w || flags[1];
+    if (walk) {
+        if (w) CM_TRY(fill_zero(ctx, q, 256));
+        CM_TRY(run(n <= 2048 ? 512 : 1024, 0));
+    }
+    count(CM_CNT_CG_WALK, walk || flags[2]);
+    CM_REQUIRE(!flags[0], CM_E_ARG, "resident CG: a row pointer or column index lies outside the %d x %d matrix", n, n);
     auto t1 = std::chrono::steady_clock::now();
     if (iters_out) *iters_out = hi;
     if (err_out) *err_out = (double)he;
     if (stats) {
         stats->path_used = CM_CG_RESIDENT;
-        stats->launches = 2;
+        stats->launches = 2 + (w && walk ? 2 : 0);
         stats->seconds = std::chrono::duration<double>(t1 - t0).count();
     }
     return CM_OK;
@@ -667,12 +741,35 @@ void graph_cache_drop(cm_ctx_t ctx)
     }
 }
 
-static int batched_launch(cm_ctx_t ctx, int nsys, const int* row_off, int total_nnz, const int* JA, const int* IA,
-                          const float* vals, const float* b, float* x, float tol, int max_iter, int* iters,
-                          float* errors, int bs, const BatchedPlan& plan, void* order_dev, void* queue_dev,
-                          int gpc = 0)
+static int default_bs(int nmax, bool walk)
 {
-    CM_TRY(fill_zero(ctx, queue_dev, 256));
+    if (nmax <= 2048) return 256;
+    if (nmax <= (walk ? 8192 : 9216)) return 512;
+    return 1024;
+}
+
+// How a batch is launched: the register form's diagonals (0: every system
+// walks) and both kernels' threads.
+struct BatchedShape {
+    int w, bs, walk_bs, gpc;
+};
+// block_size: 0 for the default, or the caller's or the autotuner's choice
+static BatchedShape batched_shape(const BatchedPlan& plan, int block_size, int gpc)
+{
+    BatchedShape S;
+    S.bs = block_size ? block_size : default_bs(plan.nmax, false);
+    S.walk_bs = block_size ? block_size : default_bs(plan.nmax, true);
+    S.w = resident_diagonals<float>(S.bs, plan.nmax, plan.nnz_mean);
+    S.gpc = gpc;
+    return S;
+}
+
+// The systems of one batch. queue_dev: 256 bytes; order_dev: nsys ints, and
+// nsys more for the systems that the register form leaves.
+static ResidentArgs<float> batched_args(int nsys, const int* row_off, int total_nnz, const int* JA, const int* IA,
+                                        const float* vals, const float* b, float* x, float tol, int max_iter,
+                                        int* iters, float* errors, void* order_dev, void* queue_dev)
+{
     ResidentArgs<float> A{};
     A.nsys = nsys;
     A.row_off = row_off;
@@ -689,15 +786,39 @@ static int batched_launch(cm_ctx_t ctx, int nsys, const int* row_off, int total_
     A.iters_out = iters;
     A.err_out = errors;
     A.queue = (unsigned*)queue_dev;
+    A.walk = (int*)order_dev + nsys;
     A.nnz_total = total_nnz;
-    return launch_resident<float>(ctx, A, plan.nmax, bs, 0, plan.nnz_mean, gpc);
+    return A;
 }
 
-static int default_bs(int nmax)
+// Queues the first launch (graph-capturable).
+static int batched_launch(cm_ctx_t ctx, const ResidentArgs<float>& A, const BatchedPlan& plan, const BatchedShape& S)
 {
-    if (nmax <= 2048) return 256;
-    if (nmax <= 9216) return 512;
-    return 1024;
+    CM_TRY(fill_zero(ctx, A.queue, 256));
+    return launch_resident<float>(ctx, A, plan.nmax, S.w ? S.bs : S.walk_bs, 0, S.w, S.gpc);
+}
+
+// Waits for it, and has the walking kernel solve the systems it left. bad:
+// some system's pattern leaves its own rows.
+static int batched_finish(cm_ctx_t ctx, ResidentArgs<float> A, const BatchedPlan& plan, const BatchedShape& S, bool& bad)
+{
+    unsigned flags[3] = {0, 0, 0};
+    auto wait = [&]() {
+        CM_HIP(hipMemcpyAsync(flags, A.queue + 1, sizeof(flags), hipMemcpyDeviceToHost, ctx->stream));
+        return ::cm::host_sync(ctx);
+    };
+    CM_TRY(wait());
+    bad = flags[0] != 0;
+    const int left = S.w ? (int)flags[1] : 0;
+    count(CM_CNT_CG_WALK, S.w ? left + (int)flags[2] : A.nsys);
+    if (left == 0) return CM_OK;
+    A.order = A.walk;
+    A.nsys = left;
+    CM_TRY(fill_zero(ctx, A.queue, 256));
+    CM_TRY(launch_resident<float>(ctx, A, plan.nmax, S.walk_bs, 0, 0, S.gpc));
+    CM_TRY(wait());
+    bad = bad || flags[0] != 0;
+    return CM_OK;
 }
 
 // ============================================ mixed precision + FP64 refinement
@@ -876,31 +997,31 @@ int cm_pcg_batched_solve(cm_ctx_t ctx, int nsys, const int* row_off, int total_r
         if (it != cm::g_tuned_bs.end()) {
             block_size = it->second.first;
             gpc = it->second.second;
-        } else {
-            block_size = cm::default_bs(plan.nmax);
         }
     }
-    unsigned bad = 0;
+    const cm::BatchedShape S = cm::batched_shape(plan, block_size, gpc);
+    bool bad = false;
     if (!use_graph) {
         cm::Temps tmp(ctx);
         void *ord, *q;
-        CM_TRY(tmp.get(sizeof(int) * nsys, &ord));
+        CM_TRY(tmp.get(2 * sizeof(int) * nsys, &ord));
         CM_TRY(tmp.get(256, &q));
         CM_HIP(hipMemcpyAsync(ord, plan.order.data(), sizeof(int) * nsys, hipMemcpyHostToDevice, ctx->stream));
-        CM_TRY(cm::batched_launch(ctx, nsys, row_off, total_nnz, JA, IA, vals, b, x, tol, max_iter, iterations,
-                                  errors, block_size, plan, ord, q, gpc));
-        CM_HIP(hipMemcpyAsync(&bad, (unsigned*)q + 1, sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
-        CM_TRY(::cm::host_sync(ctx));
+        const auto A = cm::batched_args(nsys, row_off, total_nnz, JA, IA, vals, b, x, tol, max_iter, iterations, errors,
+                                        ord, q);
+        CM_TRY(cm::batched_launch(ctx, A, plan, S));
+        CM_TRY(cm::batched_finish(ctx, A, plan, S, bad));
     } else {
         // graph path: the (queue reset + persistent solve) pair is captured
-        // once per argument set and replayed
+        // once per argument set and replayed; systems that the register form
+        // leaves are solved behind it
         cm::GraphKey key;
         memset(&key, 0, sizeof(key));
         key.ctx = ctx;
         const void* ps[9] = {row_off, JA, IA, vals, b, x, iterations, errors, nullptr};
         memcpy(key.ptrs, ps, sizeof(ps));
         key.nsys = nsys;
-        key.bs = block_size;
+        key.bs = S.bs;
         key.gpc = gpc;
         key.max_iter = max_iter;
         key.nmax = plan.nmax;
@@ -921,7 +1042,7 @@ int cm_pcg_batched_solve(cm_ctx_t ctx, int nsys, const int* row_off, int total_r
                 cm::g_graphs.erase(lru);
             }
             cm::GraphEntry ge;
-            CM_TRY(cm::dalloc(ctx, sizeof(int) * nsys, &ge.order));
+            CM_TRY(cm::dalloc(ctx, 2 * sizeof(int) * nsys, &ge.order));
             int s0 = cm::dalloc(ctx, 256, &ge.queue);
             if (s0 != CM_OK) {
                 cm::graph_release(ge);
@@ -933,17 +1054,20 @@ int cm_pcg_batched_solve(cm_ctx_t ctx, int nsys, const int* row_off, int total_r
                                ctx->stream) != hipSuccess)
                 s = cm::fail(CM_E_HIP, "batched CG: upload of the solve order failed");
             // the kernel attribute must be set outside capture
-            if (s == CM_OK)
-                s = cm::batched_launch(ctx, 0, row_off, total_nnz, JA, IA, vals, b, x, tol, max_iter, iterations,
-                                       errors, block_size, plan, ge.order, ge.queue, gpc);
+            auto A = cm::batched_args(nsys, row_off, total_nnz, JA, IA, vals, b, x, tol, max_iter, iterations, errors,
+                                      ge.order, ge.queue);
+            if (s == CM_OK) {
+                A.nsys = 0;
+                s = cm::batched_launch(ctx, A, plan, S);
+                A.nsys = nsys;
+            }
             if (s == CM_OK && ::cm::host_sync(ctx) != CM_OK)
                 s = cm::fail(CM_E_HIP, "batched CG: stream synchronization failed");
             if (s == CM_OK) {
                 if (hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
                     s = cm::fail(CM_E_HIP, "batched CG: stream capture failed to start");
                 } else {
-                    s = cm::batched_launch(ctx, nsys, row_off, total_nnz, JA, IA, vals, b, x, tol, max_iter,
-                                           iterations, errors, block_size, plan, ge.order, ge.queue, gpc);
+                    s = cm::batched_launch(ctx, A, plan, S);
                     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
                     if (s == CM_OK && e != hipSuccess)
                         s = cm::fail(CM_E_HIP, "batched CG: capture failed: %s", hipGetErrorString(e));
@@ -961,9 +1085,10 @@ int cm_pcg_batched_solve(cm_ctx_t ctx, int nsys, const int* row_off, int total_r
         it->second.last_use = ++cm::g_graph_clock;
         CM_HIP(hipGraphLaunch(it->second.exec, ctx->stream));
         cm::count(CM_CNT_KERNEL_LAUNCH, 2);
-        CM_HIP(hipMemcpyAsync(&bad, (unsigned*)it->second.queue + 1, sizeof(unsigned), hipMemcpyDeviceToHost,
-                              ctx->stream));
-        CM_TRY(::cm::host_sync(ctx));
+        CM_TRY(cm::batched_finish(ctx,
+                                  cm::batched_args(nsys, row_off, total_nnz, JA, IA, vals, b, x, tol, max_iter, iterations,
+                                                   errors, it->second.order, it->second.queue),
+                                  plan, S, bad));
     }
     CM_REQUIRE(!bad, CM_E_ARG,
                "batched CG: a system's row pointers or column indices leave its own rows (those systems report "
@@ -987,8 +1112,10 @@ int cm_pcg_batched_autotune(cm_ctx_t ctx, int nsys, const int* row_off, int tota
     CM_TRY(tmp.get(sizeof(float) * (size_t)total_rows, &xs));
     CM_TRY(tmp.get(sizeof(int) * nsys, &it));
     CM_TRY(tmp.get(sizeof(float) * nsys, &er));
-    CM_TRY(tmp.get(sizeof(int) * nsys, &ord));
+    CM_TRY(tmp.get(2 * sizeof(int) * nsys, &ord));
     CM_TRY(tmp.get(256, &q));
+    const auto A = cm::batched_args(nsys, row_off, total_nnz, JA, IA, vals, b, (float*)xs, tol, max_iter, (int*)it,
+                                    (float*)er, ord, q);
     CM_HIP(hipMemcpyAsync(ord, plan.order.data(), sizeof(int) * nsys, hipMemcpyHostToDevice, ctx->stream));
     hipEvent_t e0, e1;
     CM_HIP(hipEventCreate(&e0));
@@ -1000,14 +1127,16 @@ int cm_pcg_batched_autotune(cm_ctx_t ctx, int nsys, const int* row_off, int tota
     const int cands[3] = {256, 512, 1024};
     const int gpcs[3] = {1, 2, 4};
     int status = CM_OK;
+    bool bad = false;
     for (int c = 0; c < 9 && status == CM_OK; ++c) {
         const int bs = cands[c / 3], gpc = gpcs[c % 3];
         if ((plan.nmax + bs - 1) / bs > (bs <= 512 ? 32 : 16)) continue;  // register tile too large
         float ms_min = 1e30f;
         for (int rep = 0; rep < 2 && status == CM_OK; ++rep) {
             if (hipEventRecord(e0, ctx->stream) != hipSuccess) { status = cm::fail(CM_E_HIP, "autotune: event"); break; }
-            status = cm::batched_launch(ctx, nsys, row_off, total_nnz, JA, IA, vals, b, (float*)xs, tol, max_iter,
-                                        (int*)it, (float*)er, bs, plan, ord, q, gpc);
+            const cm::BatchedShape S = cm::batched_shape(plan, bs, gpc);
+            status = cm::batched_launch(ctx, A, plan, S);
+            if (status == CM_OK) status = cm::batched_finish(ctx, A, plan, S, bad);
             if (status != CM_OK) break;
             float ms = 0;
             if (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
@@ -1023,9 +1152,6 @@ int cm_pcg_batched_autotune(cm_ctx_t ctx, int nsys, const int* row_off, int tota
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     CM_TRY(status);
-    unsigned bad = 0;
-    CM_HIP(hipMemcpyAsync(&bad, (unsigned*)q + 1, sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
-    CM_TRY(::cm::host_sync(ctx));
     CM_REQUIRE(!bad, CM_E_ARG, "autotune: a system's row pointers or column indices leave its own rows");
     CM_REQUIRE(best > 0, CM_E_UNSUPPORTED, "autotune: no launch shape fits systems of %d rows", plan.nmax);
     {

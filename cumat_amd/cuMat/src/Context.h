@@ -77,7 +77,8 @@ public:
         JitCompile = CM_CNT_JIT_COMPILE,
         JitLaunch = CM_CNT_JIT_LAUNCH,
         CgLayout = CM_CNT_CG_LAYOUT,
-        CgDiagonals = CM_CNT_CG_DIAGONALS
+        CgDiagonals = CM_CNT_CG_DIAGONALS,
+        CgWalk = CM_CNT_CG_WALK
     };
     static Profiling& instance()
     {

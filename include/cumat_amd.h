@@ -100,7 +100,10 @@ enum cm_counter {
      * diagonals, and those whose iterations then ran over that layout */
     CM_CNT_CG_LAYOUT = 12,
     CM_CNT_CG_DIAGONALS = 13,
-    CM_CNT_COUNT = 14
+    /* no reference counterpart: systems that the one-workgroup solves walked
+     * row by row instead of keeping their matrix in registers */
+    CM_CNT_CG_WALK = 14,
+    CM_CNT_COUNT = 15
 };
 
 typedef struct cm_context* cm_ctx_t;
