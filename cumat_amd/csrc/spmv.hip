@@ -145,7 +145,7 @@ __global__ __launch_bounds__(SPMV_BS) void csr_spmv_wide_kernel(int rows, int co
         if (wave_reduce<OpMax>(re - rb) <= SPMV_ROW_MAX)
             chunk_windows<VT, T, SPMV_EPT, NB>(s, e, rb, re, IA, v, xg, slice, acc);
         else
-            chunk_rows<VT, T, NB>(r0, nr, JA, IA, v, xg, acc);
+            chunk_rows<VT, T, NB>(nr, rb, re, IA, v, xg, acc);
         if (lane < nr) {
 #pragma unroll
             for (int b = 0; b < NB; ++b) {

@@ -68,6 +68,20 @@ def test_vectors_together(gpu, batches, mean):
     check(gpu, lengths, 1000, np.int32 if batches % 2 else np.float32, batches=batches)
 
 
+@pytest.mark.parametrize("batches", [2, 3, 4])
+@pytest.mark.parametrize("mean", [4, 12])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.int32])
+def test_long_rows_and_vectors_together(gpu, batches, mean, dtype):
+    """Chunks that go row by row for all vectors of a group: both sides of a
+    wavefront and of four, a few entries to thousands."""
+    rows = 64 * 16384 // batches + 3
+    lengths = np.full(rows, mean, np.int64)
+    lengths[64 * np.arange(12) + np.arange(12)] = [129, 255, 256, 257, 320, 511, 512, 513, 575, 1000, 1024, 4097]
+    lengths[64 * 20: 64 * 21] = 300  # every row of a chunk
+    lengths[-2:] = [700, 0]
+    check(gpu, lengths, 1000, dtype, batches=batches, mode=gpu.capi.ADD if batches == 3 else 0)
+
+
 def test_shared_vector_and_bf16_values(gpu):
     cm = gpu
     check(cm, [20] * 3000, 3000, np.float32, batches=3, shared_x=False)
