@@ -11,6 +11,7 @@
 #include "spmv_wave.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 namespace cm {
@@ -110,25 +111,37 @@ __global__ __launch_bounds__(SPMV_BS, sizeof(T) == 4 ? 8 : 4) void csr_spmv_mult
 // Rows of more than SPMV_EPT entries on average: every chunk of 64 rows is
 // taken in windows of SPMV_EPT * 64 entries. Chunks with a row of more than
 // SPMV_ROW_MAX entries go row by row: one lane would add such a row while the
-// others wait.
+// others wait, and beyond 64 entries its error would exceed the row by row
+// form's (chunk_windows).
 //
 // Row by row, a row of 27 entries is one load per lane, 37 lanes idle, and a
 // wave reduction; the next row's loads wait for it. Measured on MI355X, us, row
 // by row / windows: 27 points, 572 k rows, FP64 136 / 45.5 (one vector), 332 /
-// 71.8 (three, the windows read once for all), FP32 107 / 34.1; 200 k rows of 1
+// 68.1 (three, the windows read once for all), FP32 107 / 34.1; 200 k rows of 1
 // to 39 entries FP32 41.5 / 19.3. Without the next window's loads in flight
 // 54.8, 78.8, 46.5 and 23.8.
-constexpr int SPMV_ROW_MAX = 128;
+//
+// A window holds 512 / L rows of L entries, so that many lanes add while the
+// others wait: with L the windows' instructions grow, and once the wavefronts
+// fill the chip (SPMV_CROWD) those count. Us, row by row / windows, one vector
+// of 400 k rows: FP32 L = 32 63 / 60, 40 73 / 71, 48 83 / 88, 64 106 / 123; FP64 48
+// 127 / 115. Three vectors apart, 5.4 M entries: FP32 27 91 / 64, 32 60 / 65, 48 55 /
+// 72, FP64 40 104 / 92, 48 96 / 94, 64 62 / 88. Hence the limits on a chunk's mean.
+// Fewer wavefronts wait for memory (one vector of 5.4 M entries FP32 48 38 / 26),
+// and vectors together share the loads (three of 400 k rows FP32 48 234 / 170).
+constexpr int SPMV_ROW_MAX = 64;
+constexpr long long SPMV_CROWD = 3072;
+template <typename T> constexpr int SPMV_CROWD_MEAN = sizeof(T) == 8 ? 44 : 30;
 template <typename VT, typename T, int NB>
 __global__ __launch_bounds__(SPMV_BS) void csr_spmv_wide_kernel(int rows, int cols, int nnz, int batches,
                                                                 const int* __restrict__ JA,
                                                                 const int* __restrict__ IA,
                                                                 const VT* __restrict__ vals, int vals_batched,
                                                                 const T* __restrict__ x, int x_batched,
-                                                                T* __restrict__ y, int mode)
+                                                                T* __restrict__ y, int mode, int window_max)
 {
     constexpr int WPB = SPMV_BS / 64;
-    __shared__ T lds[WPB][SPMV_EPT * 64];
+    __shared__ T lds[WPB][SPMV_EPT * 64 + 8];
     T* slice = lds[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
     const int b0 = blockIdx.y * NB;
@@ -142,7 +155,7 @@ __global__ __launch_bounds__(SPMV_BS) void csr_spmv_wide_kernel(int rows, int co
         const int s = JA[r0], e = JA[r0 + nr];
         const int rb = lane < nr ? JA[r0 + lane] : 0, re = lane < nr ? JA[r0 + lane + 1] : 0;
         T acc[NB];
-        if (wave_reduce<OpMax>(re - rb) <= SPMV_ROW_MAX)
+        if (e - s <= window_max && wave_reduce<OpMax>(re - rb) <= SPMV_ROW_MAX)
             chunk_windows<VT, T, SPMV_EPT, NB>(s, e, rb, re, IA, v, xg, slice, acc);
         else
             chunk_rows<VT, T, NB>(nr, rb, re, IA, v, xg, acc);
@@ -288,7 +301,7 @@ static int launch_csr(cm_ctx_t ctx, int rows, int cols, int nnz, int batches, co
     const bool wide = nnz > (long long)SPMV_EPT * rows;
 #define CM_WIDE(NB)                                                                                             \
     csr_spmv_wide_kernel<VT, T, NB><<<dim3(g, (batches + NB - 1) / NB), SPMV_BS, 0, ctx->stream>>>(             \
-        rows, cols, nnz, batches, JA, IA, (const VT*)vals, vb, (const T*)x, xb, (T*)y, mode)
+        rows, cols, nnz, batches, JA, IA, (const VT*)vals, vb, (const T*)x, xb, (T*)y, mode, window_max)
 #define CM_MULTI(NB)                                                                                            \
     csr_spmv_multi_kernel<VT, T, NB><<<dim3(g, (batches + NB - 1) / NB), SPMV_BS, 0, ctx->stream>>>(            \
         rows, cols, batches, JA, IA, (const VT*)vals, (const T*)x, (T*)y, mode)
@@ -296,6 +309,7 @@ static int launch_csr(cm_ctx_t ctx, int rows, int cols, int nnz, int batches, co
     // groups still fill the chip (a wavefront takes 64 rows)
     const long long waves = (long long)div_up(rows, 64) * batches;
     const int nb = (vb || !xb || waves < SPMV_MULTI_WAVES) ? 1 : std::min(batches, 4);
+    const int window_max = nb == 1 && waves >= SPMV_CROWD ? SPMV_CROWD_MEAN<T> * 64 : INT_MAX;
     if (nb == 1 && wide) CM_WIDE(1);
     else if (nb == 1)
         csr_spmv_kernel<VT, T><<<dim3(g, batches), SPMV_BS, 0, ctx->stream>>>(

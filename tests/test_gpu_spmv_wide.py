@@ -96,9 +96,40 @@ def test_shared_vector_and_bf16_values(gpu):
     assert np.all(np.abs(got - want) <= 2.0 ** -23 * 22 * size)
 
 
+@pytest.mark.parametrize("dtype,limit", [(np.int32, 30), (np.float64, 44)])
+def test_crowded_windows(gpu, dtype, limit):
+    """Both sides of the limit on a chunk's mean where the wavefronts fill the chip."""
+    lengths = np.full(64 * 3072, limit, np.int64)
+    lengths[:64 * 1000: 64] += 1
+    check(gpu, lengths, 500, dtype)
+
+
+@pytest.mark.parametrize("length", [9, 20, 27, 32, 39, 48, 64])
+@pytest.mark.parametrize("signs", [False, True])
+def test_windows_lose_no_precision(gpu, length, signs):
+    """The rms error of 20000 rows is no larger than row by row: a product per
+    lane and the wavefront's tree, emulated here. 3 % for the sampling."""
+    cm = gpu
+    rows, cols, f = 20000, 4000, np.float32
+    rng = np.random.default_rng(length)
+    draw = rng.standard_normal if signs else rng.random
+    JA = (np.arange(rows + 1) * length).astype(np.int32)
+    IA = rng.integers(0, cols, rows * length).astype(np.int32)
+    V, x = draw(IA.size).astype(f), draw(cols).astype(f)
+    A = cm.SparseMatrix.from_csr(rows, cols, JA, IA, V)
+    got = A.matvec(cm.DeviceArray.from_numpy(x)).numpy().reshape(-1)
+    lanes = np.zeros((rows, 64), f)
+    lanes[:, :length] = (V * x[IA]).reshape(rows, length)
+    while lanes.shape[1] > 1:
+        lanes = lanes[:, 0::2] + lanes[:, 1::2]
+    terms = (V.astype(np.float64) * x[IA]).reshape(rows, length)
+    rms = lambda y: np.sqrt(np.mean(((y - terms.sum(1)) / np.abs(terms).sum(1)) ** 2))
+    assert rms(got) <= 1.03 * rms(lanes[:, 0])
+
+
 @pytest.mark.parametrize("batches", [1, 2, 3, 5])
 @pytest.mark.parametrize("width", [3, 8, 9, 27])
-@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32])
 def test_ell_vectors_together(gpu, batches, width, dtype):
     """ELLPACK with padding, past the rule for groups of vectors: integer data, exact in every type."""
     cm = gpu
