@@ -186,8 +186,13 @@ __device__ __forceinline__ float dia_value<unsigned short, float>(unsigned short
 
 // tmp = A p for NB consecutive batches that share the values, and their
 // per-block partial p.tmp. A lane takes U rows CG_DIA_BS apart, so every load
-// of a wavefront is 64 consecutive elements. D: the diagonals at compile time
-// (0: A.count of them).
+// of a wavefront is 64 consecutive elements. D: the diagonals at compile time,
+// or -CH for A.count of them in CH chains. Up to 8 entries the CSR product adds a
+// row in one chain, and so does this; longer rows it adds in a wavefront's tree,
+// and here the diagonals go round four chains, from 27 on eight (rms error in eps
+// of the terms' magnitudes, uniform FP32 terms, CSR / one chain / four or eight:
+// 13 diagonals 0.343 / 0.471 / 0.331, 21 0.362 / 0.598 / 0.346, 27 0.336 / 0.653 /
+// 0.327, 32 0.343 / 0.698 / 0.339).
 //
 // Bound by the bytes: (values + p + Ap) of 160^3 with 7 diagonals are 148 MB.
 // Measured on MI355X, us per launch, CSR product -> this one: 160^3 FP32
@@ -199,6 +204,7 @@ __device__ __forceinline__ float dia_value<unsigned short, float>(unsigned short
 // 4): 160^3 73.6 / 73.5 / 72.3; 512^2 x 8 40.4 / 39.8 / 40.4; 16 x 256^2 41.9 /
 // 42.8 / 43.9: four pay where a block still has several steps to take. Two
 // batches per thread against one: 0.5 % of a solve; four: slower.
+inline int cg_dia_chains(int count) { return count <= 8 ? 1 : (count <= 26 ? 4 : 8); }
 template <typename VT, typename T, int D, int U, int NB>
 __global__ __launch_bounds__(CG_DIA_BS) void cg_dia_kernel(int n, const DiaArgs A, const VT* __restrict__ dia,
                                                            const T* __restrict__ p, T* __restrict__ tmp,
@@ -217,7 +223,9 @@ __global__ __launch_bounds__(CG_DIA_BS) void cg_dia_kernel(int n, const DiaArgs 
     const VT* db = dia + blockIdx.y * A.bstride;
     const T* pb = p + (long long)b0 * n;
     T* tb = tmp + (long long)b0 * n;
-    const int cnt = D ? D : A.count;
+    constexpr int CH = D > 0 ? 1 : -D;          // chains of a row
+    constexpr int STEP = CH > 4 ? CH : 4;       // diagonals whose loads are in flight together
+    const int cnt = D > 0 ? D : A.count;
     T s[NB];
 #pragma unroll
     for (int q = 0; q < NB; ++q) s[q] = T(0);
@@ -228,36 +236,51 @@ __global__ __launch_bounds__(CG_DIA_BS) void cg_dia_kernel(int n, const DiaArgs 
         const bool inside = first + A.off[0] >= 0 && first + CG_DIA_BS * U + A.off[cnt - 1] <= n &&
                             first + CG_DIA_BS * U <= n;
         if (inside) {
-            T acc[NB][U];
+            T acc[NB][U][CH];
 #pragma unroll
             for (int q = 0; q < NB; ++q)
 #pragma unroll
-                for (int u = 0; u < U; ++u) acc[q][u] = T(0);
-            auto add = [&](int d) {
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int k = 0; k < CH; ++k) acc[q][u][k] = T(0);
+            auto add = [&](int d, int k) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const T a = dia_value<VT, T>(db[d * A.ld + i + u * CG_DIA_BS]);
 #pragma unroll
                     for (int q = 0; q < NB; ++q)
-                        acc[q][u] += a * pb[(long long)q * n + i + u * CG_DIA_BS + A.off[d]];
+                        acc[q][u][k] += a * pb[(long long)q * n + i + u * CG_DIA_BS + A.off[d]];
                 }
             };
             if constexpr (D > 0) {
 #pragma unroll
-                for (int d = 0; d < D; ++d) add(d);
+                for (int d = 0; d < D; ++d) add(d, 0);
             } else {
-#pragma unroll 4
-                for (int d = 0; d < cnt; ++d) add(d);
+                int d = 0;
+                for (; d + STEP <= cnt; d += STEP)
+#pragma unroll
+                    for (int k = 0; k < STEP; ++k) add(d + k, k % CH);
+#pragma unroll
+                for (int k = 0; k < STEP - 1; ++k)
+                    if (d + k < cnt) add(d + k, k % CH);
             }
+#pragma unroll
+            for (int h = CH / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int q = 0; q < NB; ++q)
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int k = 0; k < h; ++k) acc[q][u][k] += acc[q][u][k + h];
 #pragma unroll
             for (int q = 0; q < NB; ++q)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const long long row = i + u * CG_DIA_BS;
                     const T own = pb[(long long)q * n + row];
-                    if (diag) acc[q][u] += diag[row] * own;
-                    tb[(long long)q * n + row] = acc[q][u];
-                    s[q] += own * acc[q][u];
+                    if (diag) acc[q][u][0] += diag[row] * own;
+                    tb[(long long)q * n + row] = acc[q][u][0];
+                    s[q] += own * acc[q][u][0];
                 }
         } else {
             for (int u = 0; u < U; ++u) {
@@ -265,12 +288,23 @@ __global__ __launch_bounds__(CG_DIA_BS) void cg_dia_kernel(int n, const DiaArgs 
                 if (row >= n) break;
 #pragma unroll
                 for (int q = 0; q < NB; ++q) {
-                    T acc = T(0);
-                    for (int d = 0; d < cnt; ++d) {
-                        // a slot the row does not store holds 0: any p of this vector will do
-                        const long long col = min(max(row + A.off[d], 0ll), (long long)n - 1);
-                        acc += dia_value<VT, T>(db[d * A.ld + row]) * pb[(long long)q * n + col];
-                    }
+                    T chain[CH];
+#pragma unroll
+                    for (int k = 0; k < CH; ++k) chain[k] = T(0);
+                    for (int d0 = 0; d0 < cnt; d0 += CH)
+#pragma unroll
+                        for (int k = 0; k < CH; ++k) {
+                            const int d = d0 + k;
+                            if (d >= cnt) break;
+                            // a slot the row does not store holds 0: any p of this vector will do
+                            const long long col = min(max(row + A.off[d], 0ll), (long long)n - 1);
+                            chain[k] += dia_value<VT, T>(db[d * A.ld + row]) * pb[(long long)q * n + col];
+                        }
+#pragma unroll
+                    for (int h = CH / 2; h > 0; h /= 2)
+#pragma unroll
+                        for (int k = 0; k < h; ++k) chain[k] += chain[k + h];
+                    T acc = chain[0];
                     const T own = pb[(long long)q * n + row];
                     if (diag) acc += diag[row] * own;
                     tb[(long long)q * n + row] = acc;
@@ -306,15 +340,19 @@ template <typename VT, typename T>
 static void launch_cg_dia(hipStream_t stream, int n, int B, int G, const DiaArgs& A, const VT* dia, const T* p, T* tmp,
                           T* part, CgState<T>* st, const T* diag)
 {
+    const int chains = cg_dia_chains(A.count);
+#define CM_DIA(U)                                                                                              \
+    if (A.count == 5) launch_cg_dia_u<VT, T, 5, U>(stream, n, B, G, A, dia, p, tmp, part, st, diag);           \
+    else if (A.count == 7) launch_cg_dia_u<VT, T, 7, U>(stream, n, B, G, A, dia, p, tmp, part, st, diag);      \
+    else if (chains == 1) launch_cg_dia_u<VT, T, -1, U>(stream, n, B, G, A, dia, p, tmp, part, st, diag);      \
+    else if (chains == 4) launch_cg_dia_u<VT, T, -4, U>(stream, n, B, G, A, dia, p, tmp, part, st, diag);      \
+    else launch_cg_dia_u<VT, T, -8, U>(stream, n, B, G, A, dia, p, tmp, part, st, diag)
     if (n >= CG_DIA_U4_ROWS) {
-        if (A.count == 5) launch_cg_dia_u<VT, T, 5, 4>(stream, n, B, G, A, dia, p, tmp, part, st, diag);
-        else if (A.count == 7) launch_cg_dia_u<VT, T, 7, 4>(stream, n, B, G, A, dia, p, tmp, part, st, diag);
-        else launch_cg_dia_u<VT, T, 0, 4>(stream, n, B, G, A, dia, p, tmp, part, st, diag);
+        CM_DIA(4);
     } else {
-        if (A.count == 5) launch_cg_dia_u<VT, T, 5, 2>(stream, n, B, G, A, dia, p, tmp, part, st, diag);
-        else if (A.count == 7) launch_cg_dia_u<VT, T, 7, 2>(stream, n, B, G, A, dia, p, tmp, part, st, diag);
-        else launch_cg_dia_u<VT, T, 0, 2>(stream, n, B, G, A, dia, p, tmp, part, st, diag);
+        CM_DIA(2);
     }
+#undef CM_DIA
 }
 
 }  // namespace cm
