@@ -276,11 +276,14 @@ __global__ __launch_bounds__(64 * NW) void col_combine_kernel(const T* __restric
 // rows at once, lane = row * Q + q, so most lanes work; the rows' results are
 // combined in LDS by halves. Lanes of col_kernel beyond Q idle: 8 x 60000 x 64
 // FP32 over columns 162 -> 25 us, over columns and batches 376 -> 30.
-// rms error in eps of the sum, uniform FP32 terms, emulated, col_kernel -> this:
-// 4096 batches of 255 rows 0.41 -> 0.35, 1000 rows 0.55 -> 0.28 (Q = 2); one
-// batch of 8000 rows 1.21 -> 0.35 (Q = 2). Not smaller everywhere: one batch of
-// 100 rows 0.32 -> 0.35, of 255 rows 0.355 -> 0.372 (Q = 32).
+// rms error in eps of the sum, emulated over FP32 terms uniform up to a random
+// scale, this against col_kernel: 4096 batches of 255 rows 0.80 to 0.88 times, one
+// batch of 700 rows 0.73 to 0.82 times. Folds of fewer than COL_NARROW_SPLIT rows
+// take at most two blocks: in more, a lane's few rows are a chain (one batch of
+// 180 rows, Q = 32, five blocks 1.04 times, two 0.94). With that 0.61 to 1.00 times
+// over 1 to 2100 batches of 64 to 700 rows and Q = 2 to 32.
 constexpr int COL_NARROW = 32;
+constexpr long long COL_NARROW_SPLIT = 512;
 template <typename Op, typename T, typename S>
 __global__ __launch_bounds__(RBS) void col_narrow_kernel(const S* __restrict__ in, int Q, long long K, long long st,
                                                          long long PS, int ksplit, T* partials, S* out)
@@ -728,7 +731,7 @@ static int run_columns(cm_ctx_t ctx, const S* in, long long P, long long Q, long
     if (Q <= COL_NARROW && K >= 64) {
         const long long per = 64 / Q;
         long long ksplit = std::max<long long>(1, (cus * 8 + P - 1) / P);
-        ksplit = std::max<long long>(1, std::min<long long>({ksplit, K / (16 * per), 1024}));
+        ksplit = std::max<long long>(1, std::min<long long>({ksplit, K / (16 * per), K < COL_NARROW_SPLIT ? 2 : 1024}));
         void* part = nullptr;
         if (ksplit > 1) CM_TRY(scratch(ctx, 1, sizeof(T) * P * ksplit * 64, &part));
         CM_REQUIRE(P * ksplit < (1ll << 31), CM_E_DIM, "reduction too large");

@@ -100,3 +100,22 @@ def test_few_kept_elements_fold_by_halves(gpu, dtype, rows, cols):
         h = (len(r) + 1) // 2
         r = [r[i] + r[i + h] if i + h < len(r) else r[i] for i in range(h)]
     assert np.array_equal(got, r[0])
+
+
+def test_few_kept_elements_of_few_batches_lose_no_precision(gpu):
+    """The rms error over 38400 folds of 180 rows is no larger than that of the
+    general kernel's order (three blocks of four wavefronts), emulated here."""
+    P, Q, K, f = 300, 32, 180, np.float32
+    errors = [[], []]
+    for seed in range(4):
+        rng = np.random.default_rng(seed)
+        # a random scale for every fold, so that no sum sits at a power of two
+        a = (rng.uniform(0, 1, (P, Q, K)) * 2 ** rng.uniform(0, 1, (P, Q, 1))).astype(f)
+        want = a.astype(np.float64).sum(axis=2)
+        x = np.moveaxis(a, 2, 0)
+        general = chain([chain([strided(x[60 * s: 60 * s + 60], w, 4) for w in range(4)]) for s in range(3)])
+        got = gpu.reduce(gpu.DeviceArray.from_numpy(a), "sum", 2).numpy(logical=True)[:, :, 0]
+        for e, y in zip(errors, (got, general)):
+            e.append((y - want) / want)
+    rms = [np.sqrt(np.mean(np.square(e))) for e in errors]
+    assert rms[0] <= rms[1]
