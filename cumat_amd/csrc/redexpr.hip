@@ -673,7 +673,7 @@ static int launch_reduce_expr(cm_ctx_t ctx, const CwProgram& P0, const RxShape& 
     bool done = false;
     {
         if (jit::want(SH.L * SH.nseg)) {
-            const int st = rx_column_launch(ctx, P, SH, rx_names<Op, T, S>(), W, spread && !W, nchunk, chunk, part, out);
+            const int st = rx_column_launch(ctx, P, SH, rx_names<Op, T, S>(), W, spread && !W, flat, nchunk, chunk, part, out);
             if (st != CM_OK && st != RX_JIT_DECLINED) return st;
             done = st == CM_OK;
         }

@@ -94,18 +94,21 @@ int units_for(long long len)
 }  // namespace
 
 // Source and key of the kernel. Shape, strides and types are constants of the
-// source, addresses and chunks are arguments.
-int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxNames& N, bool wide, bool spread, int units,
-                             std::string& key, std::string& body)
+// source, addresses, chunks and the segment count are arguments. flat (short
+// segments of a flat program): the extents are arguments as well, so that one
+// kernel serves a program of every size; element j of segment s is s * L + j.
+int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxNames& N, bool wide, bool spread, bool flat,
+                             int units, std::string& key, std::string& body)
 {
     char buf[512];
     const int V = wide ? 4 : 8;
-    key = std::string("rxcol") + (wide ? "64" : "32") + (spread ? "s" : "c") + std::to_string(units) + "|" + N.op + "|" +
+    const bool one = SH.L <= (spread ? 4 : V);
+    key = std::string(flat ? "rxcolf" : "rxcol") + (one ? "1" : "n") + (wide ? "64" : "32") + (spread ? "s" : "c") + std::to_string(units) + "|" + N.op + "|" +
           N.acc + "|" + N.store + "|k";
     // kept coordinates of the lane's segment (once), reduced coordinates of
     // element j (uniform: scalar registers)
     std::string kept, red;
-    for (int a = 0; a < SH.nk; ++a) {
+    for (int a = 0; a < SH.nk && !flat; ++a) {
         snprintf(buf, sizeof(buf), "%lld@%d,", SH.kdim[a], SH.kaxis[a]);
         key += buf;
         snprintf(buf, sizeof(buf), "    { const long long q = w_ / %lldll; k3[%d] = w_ - q * %lldll; w_ = q; }\n", SH.kdim[a],
@@ -114,7 +117,7 @@ int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxName
     }
     key += "r";
     const bool narrow = SH.L < 4294967295ll;
-    for (int a = 0; a < SH.nr; ++a) {
+    for (int a = 0; a < SH.nr && !flat; ++a) {
         snprintf(buf, sizeof(buf), "%lld@%d,", SH.rdim[a], SH.raxis[a]);
         key += buf;
         if (a + 1 == SH.nr)
@@ -138,11 +141,16 @@ int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxName
         if (L.kind != CM_LEAF_STRIDED) return RX_JIT_DECLINED;
         long long s[3];
         strides_of(L, s);
-        snprintf(buf, sizeof(buf), "L%d,%lld,%lld,%lld|", L.dtype, s[0], s[1], s[2]);
+        if (flat) snprintf(buf, sizeof(buf), "L%d%c|", L.dtype, (P.leaf_scalar >> l) & 1 ? 's' : 'd');
+        else snprintf(buf, sizeof(buf), "L%d,%lld,%lld,%lld|", L.dtype, s[0], s[1], s[2]);
         key += buf;
         const char* type = L.dtype == CM_BOOL ? "unsigned char" : (L.dtype == CM_F64 ? "uint64_t" : "uint32_t");
         std::string koff, roff;
-        for (int a = 0; a < 3; ++a) {
+        if (flat && !((P.leaf_scalar >> l) & 1)) {
+            koff = "w_ * A.L";
+            roff = "e_";
+        }
+        for (int a = 0; a < 3 && !flat; ++a) {
             if (s[a] == 0 || dim[a] <= 1) continue;
             std::string& o = is_red[a] ? roff : koff;
             snprintf(buf, sizeof(buf), "%s%s3[%d] * %lldll", o.empty() ? "" : " + ", is_red[a] ? "r" : "k", a, s[a]);
@@ -193,11 +201,10 @@ int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxName
     const int waves = units >= 4 ? units : 4, tiles = waves / units;
     snprintf(buf, sizeof(buf),
              "typedef %s TT;\ntypedef %s SS;\ntypedef %s OP;\ntypedef %s R;\n"
-             "constexpr int V = %d, PP = %d, UNITS = %d, TILES = %d;\nconstexpr long long NSEG = %lldll;\nconstexpr bool ONE = %s;\n",
-             N.acc, N.store, N.op, wide ? "uint64_t" : "uint32_t", V, pp, units, tiles, SH.nseg,
-             SH.L <= (spread ? 4 : V) ? "true" : "false");
+             "constexpr int V = %d, PP = %d, UNITS = %d, TILES = %d;\nconstexpr bool ONE = %s;\n",
+             N.acc, N.store, N.op, wide ? "uint64_t" : "uint32_t", V, pp, units, tiles, one ? "true" : "false");
     body = std::string("struct JitRxArgs { const void* leaf[") + std::to_string(CM_CWISE_MAX_LEAVES) +
-           "]; void* partials; void* out; long long L, chunk; int nchunk, pad; };\n" + buf +
+           "]; void* partials; void* out; long long L, chunk, nseg; int nchunk, pad; };\n" + buf +
            (spread ? "#define FIRST(t) ((long long)((t) >> 6) * 512 + ((t) & 63) * 4)\n"
                      "#define EL(j0, k) ((j0) + ((k) >> 2) * 256 + ((k) & 3))\n"
                    : "#define FIRST(t) ((long long)(t) * V)\n#define EL(j0, k) ((j0) + (k))\n") +
@@ -210,8 +217,8 @@ int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxName
            "    const int unit = wave % UNITS;\n"
            "    const int c = blockIdx.x % A.nchunk;\n"
            "    const long long s = ((long long)(blockIdx.x / A.nchunk) * TILES + wave / UNITS) * 64 + lane;\n"
-           "    const bool ok = s < NSEG;\n"
-           "    long long w_ = ok ? s : NSEG - 1;\n"
+           "    const bool ok = s < A.nseg;\n"
+           "    long long w_ = ok ? s : A.nseg - 1;\n"
            "    long long k3[3] = {0, 0, 0};\n" + kept + bases + scalars +
            "    const long long beg = c * A.chunk;\n"
            "    const long long end = min(A.L, beg + A.chunk);\n"
@@ -294,8 +301,21 @@ int jit_reduce_column_source(const CwProgram& P, const RxShape& SH, const RxName
     return CM_OK;
 }
 
+namespace {
+
+// JitRxArgs with the segment count
+struct JitRxColArgs {
+    const void* leaf[CM_CWISE_MAX_LEAVES];
+    void* partials;
+    void* out;
+    long long L, chunk, nseg;
+    int nchunk, pad;
+};
+
+}  // namespace
+
 int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const RxNames& N, bool wide, bool spread,
-                     long long nchunk, long long chunk, void* partials, void* out)
+                     bool flat, long long nchunk, long long chunk, void* partials, void* out)
 {
     // also many short segments, whatever their layout: a block per segment
     // costs 0.8 ns a segment with hardly a thread at work
@@ -307,17 +327,21 @@ int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const 
     if (!many_short && !rx_column_wins(P, SH)) return RX_JIT_DECLINED;
     const int units = units_for(chunk < SH.L ? chunk : SH.L);
     if ((SH.nseg + 63) / 64 * nchunk * units < MIN_WAVES) return RX_JIT_DECLINED;
+    // short segments of a flat program need no shape in the source
+    flat = flat && many_short;
     // everything the generator reads
-    std::string sig("rxcol");
+    std::string sig(flat ? "rxcolf" : "rxcol");
     sig += N.op;
     sig += N.acc;
     sig += N.store;
     jit::sig_add(sig, (int)wide);
     jit::sig_add(sig, (int)spread);
     jit::sig_add(sig, units);
+    jit::sig_add(sig, (int)(SH.L <= (spread ? 4 : (wide ? 4 : 8))));
+    jit::sig_add(sig, flat ? P.leaf_scalar : 0u);
     jit::sig_add(sig, SH.nk);
     jit::sig_add(sig, SH.nr);
-    for (int a = 0; a < 3; ++a) {
+    for (int a = 0; a < 3 && !flat; ++a) {
         jit::sig_add(sig, a < SH.nk ? SH.kdim[a] : 0ll);
         jit::sig_add(sig, a < SH.nk ? SH.kaxis[a] : -1);
         jit::sig_add(sig, a < SH.nr ? SH.rdim[a] : 0ll);
@@ -328,6 +352,7 @@ int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const 
         const cm_leaf& L = P.leaves[l];
         jit::sig_add(sig, L.dtype);
         jit::sig_add(sig, L.kind);
+        if (flat) continue;
         jit::sig_add(sig, L.sr);
         jit::sig_add(sig, L.sc);
         jit::sig_add(sig, L.sb);
@@ -347,20 +372,21 @@ int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const 
     jit::Kernel k;
     if (jit::find_sig(sig, &k) != 0) {
         std::string key, body;
-        if (jit_reduce_column_source(P, SH, N, wide, spread, units, key, body) != CM_OK) return RX_JIT_DECLINED;
+        if (jit_reduce_column_source(P, SH, N, wide, spread, flat, units, key, body) != CM_OK) return RX_JIT_DECLINED;
         if (jit::get(key, body, "cm_jit_reduce", &k) != 0) return RX_JIT_DECLINED;
         jit::put_sig(sig, k);
     }
     const int waves = units >= 4 ? units : 4, tiles = waves / units;
     const long long blocks = (SH.nseg + 64ll * tiles - 1) / (64ll * tiles) * nchunk;
     if (blocks >= (1ll << 31)) return RX_JIT_DECLINED;
-    JitRxArgs A;
+    JitRxColArgs A;
     memset(&A, 0, sizeof(A));
     for (int l = 0; l < P.nleaves; ++l) A.leaf[l] = P.leaves[l].ptr;
     A.partials = partials;
     A.out = out;
     A.L = SH.L;
     A.chunk = chunk;
+    A.nseg = SH.nseg;
     A.nchunk = (int)nchunk;
     if (jit::launch(k, (unsigned)blocks, 64 * waves, ctx->stream, &A, sizeof(A)) != 0)
         return fail(CM_E_HIP, "cm_reduce_expr: launch of the generated kernel failed");

@@ -39,8 +39,9 @@ struct RxNames {
 
 // Launches the generated reduction with lanes along the kept axes where the
 // expression's memory lies that way (rx_column_wins); RX_JIT_DECLINED
-// elsewhere. Same chunks, partials and bits as reduce_expr_kernel.
+// elsewhere. Same chunks, partials and bits as reduce_expr_kernel. flat: every
+// leaf lies in the virtual order or is a broadcast scalar (P.leaf_scalar).
 int rx_column_launch(cm_ctx_t ctx, const CwProgram& P, const RxShape& SH, const RxNames& N, bool wide, bool spread,
-                     long long nchunk, long long chunk, void* partials, void* out);
+                     bool flat, long long nchunk, long long chunk, void* partials, void* out);
 
 }  // namespace cm

@@ -8,15 +8,17 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def both(cm, fn):
+def both(cm, fn, reset=True):
     """fn's result by the interpreter and by the generated kernels."""
     out = []
     for mode in (0, 2):
         old = cm.jit_mode(mode)
         try:
-            cm.reset_counters()
+            if reset:
+                cm.reset_counters()
+            before = cm.counters()["JitLaunch"]
             out.append(fn())
-            assert cm.counters()["JitLaunch"] == mode // 2
+            assert cm.counters()["JitLaunch"] - before == mode // 2
         finally:
             cm.jit_mode(old)
     assert out[0].tobytes() == out[1].tobytes()
@@ -124,6 +126,22 @@ def test_bool_result(gpu):
     for op, ref in (("all", np.all), ("any", np.any)):
         got = both(cm, lambda: cm.reduce(A.expr() > cm.as_expr(np.float32(-2.5)), op, cm.capi.AXIS_COL).numpy(logical=True))
         assert np.array_equal(got, ref(a > -2.5, axis=2, keepdims=True))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_short_segments_share_a_kernel(gpu, dtype):
+    """A flat program's kernel serves every size: a program whose sizes change
+    compiles once."""
+    cm = gpu
+    cm.reset_counters()
+    for length, count in ((40, 40000), (41, 40001), (100, 33000), (9, 33333), (40, 40000)):
+        a, b = data((3, length, count), dtype, 11), data((3, length, count), dtype, 12)
+        A, Bv = cm.DeviceArray.from_numpy(a), cm.DeviceArray.from_numpy(b)
+        ex = (A.expr() * 1.25 - Bv).cwiseAbs2()  # a program of this test alone
+        got = both(cm, lambda: cm.reduce(ex, "sum", cm.capi.AXIS_ROW).numpy(logical=True), reset=False)
+        x = (a.astype(np.float64) * 1.25 - b) ** 2
+        assert np.all(np.abs(got - x.sum(axis=1, keepdims=True)) <= np.finfo(dtype).eps * (length + 6) * x.sum(axis=1, keepdims=True))
+    assert cm.counters()["JitCompile"] == 1
 
 
 @pytest.mark.parametrize("diagonal_first", [False, True])
