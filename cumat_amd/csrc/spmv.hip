@@ -11,16 +11,20 @@
 #include "spmv_wave.hpp"
 
 #include <algorithm>
-#include <climits>
 #include <type_traits>
 
 namespace cm {
 
 constexpr int SPMV_BS = 256;
 constexpr int SPMV_EPT = 8;   // staged non-zeros per lane (8 per row on average)
-// Vectors are multiplied together from this many (wavefronts x vectors) on:
-// below, 8 vectors of 300^2 (11 k) take 7.5 us either way.
-constexpr long long SPMV_MULTI_WAVES = 16384;
+// Vectors are multiplied together from this many (wavefronts x vectors) on; below,
+// a launch of one vector each has more loads in flight. Us, apart / together:
+// narrow rows (5 points) FP32 4 vectors of 200 k rows (12.5 k) 8.3 / 9.0, 3 of 400 k
+// (18.8 k) 10.7 / 10.6; windows (1 to 39 entries) FP32 4 of 60 k (3.8 k) 13.2 / 17.5, 3
+// of 100 k (4.7 k) 18.0 / 16.9, 8 of 60 k (7.5 k) 22.8 / 18.7, 27 points FP64 4 of 60 k
+// 17.3 / 19.0, 3 of 100 k 21.6 / 19.6; ELLPACK (a thread takes a row) with 27 slots 4
+// of 30 k (1.9 k) 12.0 / 11.5, 8 of 10 k (1.3 k) 7.3 / 9.0, 4 of 60 k (3.8 k) 13.4 / 11.8.
+constexpr long long SPMV_MULTI_WAVES = 16384, SPMV_MULTI_WIDE = 4500, ELL_MULTI_WAVES = 3072;
 
 template <typename VT, typename T>
 __global__ __launch_bounds__(SPMV_BS) void csr_spmv_kernel(int rows, int cols, int nnz,
@@ -78,7 +82,7 @@ __global__ __launch_bounds__(SPMV_BS, sizeof(T) == 4 ? 8 : 4) void csr_spmv_mult
     T* slice = lds[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
     const int b0 = blockIdx.y * NB;
-    const int nb = min(NB, batches - b0);  // a vector past the last one repeats the group's first
+    const int nb = NB == 1 ? 1 : min(NB, batches - b0);  // a vector past the last one repeats the group's first
     const VT* v = vals;
     const T* xb = x + (long long)b0 * cols;
     T* yb = y + (long long)b0 * rows;
@@ -128,7 +132,8 @@ __global__ __launch_bounds__(SPMV_BS, sizeof(T) == 4 ? 8 : 4) void csr_spmv_mult
 // 127 / 115. Three vectors apart, 5.4 M entries: FP32 27 91 / 64, 32 60 / 65, 48 55 /
 // 72, FP64 40 104 / 92, 48 96 / 94, 64 62 / 88. Hence the limits on a chunk's mean.
 // Fewer wavefronts wait for memory (one vector of 5.4 M entries FP32 48 38 / 26),
-// and vectors together share the loads (three of 400 k rows FP32 48 234 / 170).
+// and vectors together share the loads (three of 400 k rows FP32 48 234 / 172, FP64 64
+// 341 / 319).
 constexpr int SPMV_ROW_MAX = 64;
 constexpr long long SPMV_CROWD = 3072;
 template <typename T> constexpr int SPMV_CROWD_MEAN = sizeof(T) == 8 ? 44 : 30;
@@ -145,7 +150,7 @@ __global__ __launch_bounds__(SPMV_BS) void csr_spmv_wide_kernel(int rows, int co
     T* slice = lds[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
     const int b0 = blockIdx.y * NB;
-    const int nb = min(NB, batches - b0);
+    const int nb = NB == 1 ? 1 : min(NB, batches - b0);
     const VT* v = vals + (vals_batched ? (long long)b0 * nnz : 0);
     const T* xb = x + (x_batched ? (long long)b0 * cols : 0);
     T* yb = y + (long long)b0 * rows;
@@ -188,7 +193,7 @@ __global__ void ell_spmv_w_kernel(int rows, int cols, int npr, int batches, cons
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     const int b0 = blockIdx.y * NB;
-    const int nb = min(NB, batches - b0);
+    const int nb = NB == 1 ? 1 : min(NB, batches - b0);
     const T* v = vals + (vals_batched ? (long long)b0 * rows * npr : 0);
     const T* xb = x + (x_batched ? (long long)b0 * cols : 0);
     int c[MAXW];
@@ -222,7 +227,7 @@ __global__ void ell_spmv_kernel(int rows, int cols, int npr, int batches, const 
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     const int b0 = blockIdx.y * NB;
-    const int nb = min(NB, batches - b0);  // a vector past the last one repeats the group's first
+    const int nb = NB == 1 ? 1 : min(NB, batches - b0);  // a vector past the last one repeats the group's first
     const T* v = vals + (vals_batched ? (long long)b0 * rows * npr : 0);
     const T* xb = x + (x_batched ? (long long)b0 * cols : 0);
     T acc[NB];
@@ -308,8 +313,8 @@ static int launch_csr(cm_ctx_t ctx, int rows, int cols, int nnz, int batches, co
     // vectors that share the values are multiplied together, as long as the
     // groups still fill the chip (a wavefront takes 64 rows)
     const long long waves = (long long)div_up(rows, 64) * batches;
-    const int nb = (vb || !xb || waves < SPMV_MULTI_WAVES) ? 1 : std::min(batches, 4);
-    const int window_max = nb == 1 && waves >= SPMV_CROWD ? SPMV_CROWD_MEAN<T> * 64 : INT_MAX;
+    const int nb = (vb || !xb || waves < (wide ? SPMV_MULTI_WIDE : SPMV_MULTI_WAVES)) ? 1 : std::min(batches, 4);
+    const int window_max = 64 * (nb == 1 && waves >= SPMV_CROWD ? SPMV_CROWD_MEAN<T> : SPMV_ROW_MAX);
     if (nb == 1 && wide) CM_WIDE(1);
     else if (nb == 1)
         csr_spmv_kernel<VT, T><<<dim3(g, batches), SPMV_BS, 0, ctx->stream>>>(
@@ -346,7 +351,7 @@ static void launch_ell(cm_ctx_t ctx, int rows, int cols, int npr, int batches, c
                        int vb, const void* x, int xb, void* y, int mode)
 {
     // together where the groups still fill the chip (as the CSR product; a thread takes a row)
-    const bool multi = !vb && xb && (long long)rows * batches >= 64 * SPMV_MULTI_WAVES;
+    const bool multi = !vb && xb && (long long)rows * batches >= 64 * ELL_MULTI_WAVES;
     const int nb = multi ? std::min(batches, 4) : 1;
     if (nb == 4) launch_ell_nb<T, 4>(ctx, rows, cols, npr, batches, idx, vals, vb, x, xb, y, mode);
     else if (nb == 3) launch_ell_nb<T, 3>(ctx, rows, cols, npr, batches, idx, vals, vb, x, xb, y, mode);

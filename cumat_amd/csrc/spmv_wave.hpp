@@ -143,8 +143,8 @@ __device__ __forceinline__ void chunk_rows(int nr, int rb, int re, const int* __
 // that lies in the window. Row lane: entries [rb, re). slice: EPT * 64 + 8
 // elements.
 //
-// A row is added in blocks of eight, each a tree, and the blocks go round four
-// partial sums. In one chain each of four, as before, the error grew with the
+// A row is added in blocks of eight, each a tree, and a window's blocks go round
+// four partial sums. In one chain each of four, as before, the error grew with the
 // row: rms in eps of the sum of the terms' magnitudes, FP32, row by row / four
 // chains / this: uniform terms 32 entries 0.347 / 0.370 / 0.347, 64 0.347 / 0.405
 // / 0.347; normal 32 0.150 / 0.163 / 0.150, 64 0.116 / 0.145 / 0.116.
@@ -189,15 +189,21 @@ __device__ __forceinline__ void chunk_windows(int s, int end, int rb, int re, co
 #pragma unroll
             for (int j = 0; j < EPT; ++j) slice[lane + 64 * j] = Load<VT, T>::get(v, j) * xv[j];
             __builtin_amdgcn_wave_barrier();  // as in chunk_compute
-            auto add = [&](T t) {
-                const T sum = part[b][0] + t;
-#pragma unroll
-                for (int q = 0; q < 3; ++q) part[b][q] = part[b][q + 1];
-                part[b][3] = sum;
-            };
             auto four = [&](int k) { return (slice[k] + slice[k + 1]) + (slice[k + 2] + slice[k + 3]); };
             int k = a;
-            for (; k + 8 <= e; k += 8) add(four(k) + four(k + 4));
+            for (; k + 32 <= e; k += 32)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    part[b][q] += four(k + 8 * q) + four(k + 8 * q + 4);
+                    // 32 reads in flight would take the registers of a wavefront or two
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                if (k + 8 <= e) {
+                    part[b][q] += four(k) + four(k + 4);
+                    k += 8;
+                }
             if (k < e) {
                 T t = T(0);
                 if (k + 4 <= e) {
@@ -206,7 +212,7 @@ __device__ __forceinline__ void chunk_windows(int s, int end, int rb, int re, co
                 }
                 const T t0 = k < e ? slice[k] : T(0), t1 = k + 1 < e ? slice[k + 1] : T(0),
                         t2 = k + 2 < e ? slice[k + 2] : T(0);
-                add(t + ((t0 + t1) + t2));
+                part[b][3] += t + ((t0 + t1) + t2);
             }
             __builtin_amdgcn_wave_barrier();
         }

@@ -82,6 +82,15 @@ def test_long_rows_and_vectors_together(gpu, batches, mean, dtype):
     check(gpu, lengths, 1000, dtype, batches=batches, mode=gpu.capi.ADD if batches == 3 else 0)
 
 
+@pytest.mark.parametrize("rows", [64 * 1500 - 64, 64 * 1500])
+def test_rule_for_groups_of_windows(gpu, rows):
+    """Both sides of the limit from which the vectors of windows go together."""
+    lengths = np.random.default_rng(8).integers(1, 40, rows)
+    lengths[77] = 100
+    check(gpu, lengths, 1000, np.int32, batches=3)
+    check(gpu, lengths, 1000, np.float64, batches=3)
+
+
 def test_shared_vector_and_bf16_values(gpu):
     cm = gpu
     check(cm, [20] * 3000, 3000, np.float32, batches=3, shared_x=False)
