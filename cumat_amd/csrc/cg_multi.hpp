@@ -839,17 +839,17 @@ __global__ __launch_bounds__(CG_BS) void cg_iter_kernel(int n, int it, int B, in
 // the evaluation's partials has a known address, so the first rows' loads and
 // the state are requested together, before the state is looked at.
 // Measured on MI355X, us per launch at 128^2 FP32: 5.9 -> 3.8 (an empty launch
-// is 2 to 3 of them); whole iterations 9.9 -> 8.1, 360^2 10.8 -> 8.8, FP64 128^2
+// is 2 to 3 of them); whole iterations 9.9 -> 8.0 to 8.5, 360^2 10.8 -> 8.8, FP64 128^2
 // 11.3 -> 9.0, 8 right-hand sides of 128^2 13.1 -> 9.5. One element per thread in
-// KB (four times the blocks) changed nothing.
-template <typename VT, typename T, int D>
+// KB (four times the blocks) changed nothing. The two-launch form has one matrix
+// for all batches, which stop together, and no diagonal of its own (cm_pcg_solve).
+template <typename T, int D>
 __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B, int G2, const DiaArgs A,
-                                                            const VT* __restrict__ dia, const T* __restrict__ invd,
-                                                            int istride, const T* __restrict__ r,
-                                                            const T* __restrict__ pprev, T* __restrict__ pnext,
-                                                            T* __restrict__ tmp, T* __restrict__ part1,
-                                                            const T* __restrict__ part2, CgState<T>* st,
-                                                            const T* __restrict__ diag, CgMirror* __restrict__ mirror)
+                                                            const T* __restrict__ dia, const T* __restrict__ ib,
+                                                            const T* __restrict__ r, const T* __restrict__ pprev,
+                                                            T* __restrict__ pnext, T* __restrict__ tmp,
+                                                            T* __restrict__ part1, const T* __restrict__ part2,
+                                                            CgState<T>* st, CgMirror* __restrict__ mirror)
 {
     const int bb = blockIdx.y;
     __shared__ T red[2 * CG_BS / 64];
@@ -858,8 +858,6 @@ __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B
     __shared__ T q_s[CG_MAXB];
     const int lane = threadIdx.x & 63;
     const long long off = (long long)bb * n;
-    const VT* db = dia + bb * A.bstride;
-    const T* ib = invd + (long long)bb * istride;
     const T* rb = r + off;
     const T* pp = pprev + off;
     RowBlockWalk w(blockIdx.x, gridDim.x, div_up_dev(n, CG_BS));
@@ -870,7 +868,7 @@ __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B
         for (int d = 0; d < D; ++d) {
             // a slot the row does not store holds 0: any column of this vector will do
             const long long c = min(max(row + A.off[d], 0ll), (long long)n - 1);
-            val[d] = dia_value<VT, T>(db[d * A.ld + row]);
+            val[d] = dia[d * A.ld + row];
             po[d] = pp[c];
             ro[d] = rb[c];
             io[d] = ib[c];
@@ -882,13 +880,9 @@ __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B
     if (w.valid()) load();
     // ---- the state and the previous iteration's sums (as cg_iter_kernel)
     const int status = st->status;
-    const bool per_batch = st->per_batch != 0;
-    const int done_k = (lane < B && per_batch) ? st->bdone[lane] : (int)CG_RUNNING;
     const T thr_k = lane < B ? st->thr[lane] : T(0);
     const T rhs_k = lane < B ? st->rhs2[lane] : T(1);
-    const T thr_own = st->thr[bb];
     const int max_iter = st->max_iter;
-    const int own_done = per_batch ? st->bdone[bb] : (int)CG_RUNNING;
     const int prev = it - 1;
     const T absOld = st->absNew[prev & 1][bb];
     if (B == 1) {
@@ -902,39 +896,18 @@ __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B
     }
     __syncthreads();
     if (status != CG_RUNNING) return;
-    const bool own_prev = own_done != CG_RUNNING;
-    // a batch that finished earlier has nothing to do; block (0,0) still
-    // evaluates, it owns the global status
-    if (own_prev && !(blockIdx.x == 0 && bb == 0)) return;
-    const bool all = __ballot(lane < B && done_k == CG_RUNNING && !(rr_s[lane] < thr_k)) == 0;
-    const bool own_conv = own_prev || rr_s[bb] < thr_own;
+    const bool all = __ballot(lane < B && !(rr_s[lane] < thr_k)) == 0;
     if (threadIdx.x < B) q_s[lane] = rr_s[lane] / rhs_k;  // read below by thread 0, in this wavefront
     __builtin_amdgcn_wave_barrier();
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (per_batch && !own_prev) {
-            st->berr[bb] = sqrt((double)q_s[bb]);
-            if (own_conv) {
-                st->bdone[bb] = CG_CONVERGED;
-                st->biters[bb] = prev;  // the converging step is not counted
-            } else {
-                st->biters[bb] = it;
-            }
-        }
-        const bool pub = all || it >= max_iter || (prev % CG_CHUNK) == CG_CHUNK - 1;
-        if (per_batch && !own_prev && (pub || own_conv)) {
-            mirror->berr[bb] = st->berr[bb];
-            mirror->biters[bb] = st->biters[bb];
-            mirror->bdone[bb] = st->bdone[bb];
-        }
         if (bb == 0) {
-            if (!per_batch) {
-                T m = 0;
-                for (int k = 0; k < B; ++k) m = (k == 0 || q_s[k] > m) ? q_s[k] : m;
-                st->err = sqrt((double)m);
-            }
+            const bool pub = all || it >= max_iter || (prev % CG_CHUNK) == CG_CHUNK - 1;
+            T m = 0;
+            for (int k = 0; k < B; ++k) m = (k == 0 || q_s[k] > m) ? q_s[k] : m;
+            st->err = sqrt((double)m);
             if (all) {
                 st->status = CG_CONVERGED;
-                st->iters = prev;
+                st->iters = prev;  // the converging step is not counted
             } else {
                 st->iters = it;
                 if (it >= max_iter) st->status = CG_MAXIT;
@@ -946,10 +919,9 @@ __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B
                 mirror->status = st->status;
             }
         }
-        if (!(per_batch && own_conv)) st->absNew[it & 1][bb] = rz_s[bb];
+        st->absNew[it & 1][bb] = rz_s[bb];
     }
-    if (per_batch ? own_conv : all) return;
-    if (it >= max_iter) return;
+    if (all || it >= max_iter) return;
     const T beta = rz_s[bb] / absOld;
     T s = T(0);
     while (w.valid()) {
@@ -959,7 +931,6 @@ __global__ __launch_bounds__(CG_BS) void cg_dia_iter_kernel(int n, int it, int B
 #pragma unroll
             for (int d = 1; d < D; ++d) ap += val[d] * cg_pnext(beta, po[d], io[d], ro[d]);
             const T pv = cg_pnext(beta, pw, iw, rw);
-            if (diag) ap += diag[row] * pv;
             pnext[off + row] = pv;
             tmp[off + row] = ap;
             s += pv * ap;
@@ -1372,14 +1343,14 @@ struct CgBatchOpts {
     const BlockOp* block = nullptr;  // a block-CSR operator replaces the CSR matrix (FP32)
 };
 
-template <typename VT, typename T>
+template <typename T>
 static void launch_cg_dia_iter(hipStream_t stream, int n, int it, int B, int G1, int G2, const DiaArgs& A,
-                               const VT* dia, const T* invd, int istride, const T* r, const T* pprev, T* pnext, T* tmp,
-                               T* part1, const T* part2, CgState<T>* st, const T* diag, CgMirror* mirror)
+                               const T* dia, const T* invd, const T* r, const T* pprev, T* pnext, T* tmp, T* part1,
+                               const T* part2, CgState<T>* st, CgMirror* mirror)
 {
-#define CM_DIA_ITER(D)                                                                                      \
-    cg_dia_iter_kernel<VT, T, D><<<dim3(G1, B), CG_BS, 0, stream>>>(n, it, B, G2, A, dia, invd, istride, r, \
-                                                                    pprev, pnext, tmp, part1, part2, st, diag, mirror)
+#define CM_DIA_ITER(D)                                                                                         \
+    cg_dia_iter_kernel<T, D><<<dim3(G1, B), CG_BS, 0, stream>>>(n, it, B, G2, A, dia, invd, r, pprev, pnext, tmp, \
+                                                                part1, part2, st, mirror)
     if (A.count == 3) CM_DIA_ITER(3);
     else if (A.count == 5) CM_DIA_ITER(5);
     else CM_DIA_ITER(7);
@@ -1425,6 +1396,8 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
     const BlockOp* block = opt.block;
     CM_REQUIRE(!block || (invd && !opt.fused && !dense && std::is_same<T, float>::value && n == 4 * block->rows),
                CM_E_ARG, "CG: a block operator needs FP32, an inverse diagonal and the three-launch form");
+    CM_REQUIRE(!opt.fused || (same_type && !diag && !opt.vals_batched && !opt.per_batch), CM_E_ARG,
+               "CG: the two-launch form has one matrix of the vectors' type, and batches that stop together");
     CM_REQUIRE(B >= 1 && B <= CG_MAXB, CM_E_UNSUPPORTED, "CG: %d right-hand sides (max %d)", B, CG_MAXB);
     Temps tmp(ctx);
     const long long N = (long long)n * B;
@@ -1590,9 +1563,9 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
             da.bstride = vstride ? da.count * dia_ld : 0;
             for (int d = 0; d < da.count; ++d) da.off[d] = hplan->off[d];
             dia_on = &da;
-            count(CM_CNT_CG_DIAGONALS);
             if (!fused) G1 = walk_grid(div_up(n, cg_dia_rows_per_block(n)), gcap);
         }
+        if (dia_on) count(CM_CNT_CG_DIAGONALS, todo);
         for (int k = 0; k < todo; ++k, ++it) {
             if (!fused) {
                 launch_cg_iteration<VT, T>(ctx, n, B, G1, G2, JA, IA, vals, vstride, invd, istride, p, t, x, r, part1,
@@ -1601,8 +1574,9 @@ static int pcg_multikernel(cm_ctx_t ctx, int n, int nnz, int B, const int* JA, c
             }
             T* pcur = pbuf[it & 1];
             if (dia_on) {
-                launch_cg_dia_iter<VT, T>(ctx->stream, n, it, B, G1, G2, da, dia, invd, istride, r, pbuf[(it - 1) & 1],
-                                          pcur, t, part1, part2, st, diag, mirror);
+                if constexpr (same_type)
+                    launch_cg_dia_iter<T>(ctx->stream, n, it, B, G1, G2, da, dia, invd, r, pbuf[(it - 1) & 1], pcur, t,
+                                          part1, part2, st, mirror);
                 cg_update_kernel<T, true, 1, 0, true><<<dim3(G2, B), CG_BS, 0, ctx->stream>>>(
                     n, it, G1, part1, invd, istride, pcur, t, x, r, part2, st, r0);
                 continue;

@@ -97,7 +97,7 @@ enum cm_counter {
     CM_CNT_JIT_COMPILE = 10,
     CM_CNT_JIT_LAUNCH = 11,
     /* no reference counterpart: CG solves that laid their matrix out by
-     * diagonals, and those whose iterations then ran over that layout */
+     * diagonals, and iterations issued over that layout */
     CM_CNT_CG_LAYOUT = 12,
     CM_CNT_CG_DIAGONALS = 13,
     /* no reference counterpart: systems that the one-workgroup solves walked
