@@ -16,7 +16,7 @@
 // What bounds it: the bytes, each leaf once; a leaf that also appears
 // untransposed is read a second time through the caches. Measured on MI355X,
 // (A + A^T) * 0.5, us, gathering / tiled: FP32 1021 x 1021 x 61 420 -> 132
-// (3.8 TB/s), 1024 x 1024 x 64 -> 114 (4.7), 4096^2 113 -> 31, 8000^2 504 ->
+// (3.8 TB/s), 1024 x 1024 x 64 -> 82 (6.5), 4096^2 113 -> 31, 8000^2 504 ->
 // 117, 64 x 64 x 4000 42 -> 22; FP64 2048 x 2048 x 4 205 -> 61. Whole
 // batches per XCD against tiles dealt to all: 1021 x 1021 x 61 132 / 138.
 // Tiles along a diagonal: 8000^2 123 -> 146, others the same.
@@ -97,8 +97,8 @@ int jit_cwise_tile_source(const CwProgram& P, unsigned mask, bool wide, bool nt,
             lds += std::string("    __shared__ ") + word + " t" + n + "[TILE * PITCH];\n";
             stage += std::string("    ") + word + " g" + n + "[PER];\n";
             snprintf(buf, sizeof(buf),
-                     "    { const %s* p = (const %s*)A.leaf[%d] + b * %lldll + (s0 + lane);\n#pragma unroll\n"
-                     "      for (int k = 0; k < PER; ++k) g%d[k] = (s0 + lane < S && f0 + w + 4 * k < F)"
+                     "    { const %s* p = (const %s*)A.leaf[%d] + b * %lldll + (ts0 + lane);\n#pragma unroll\n"
+                     "      for (int k = 0; k < PER; ++k) g%d[k] = (ts0 + lane < S && f0 + w + 4 * k < F)"
                      " ? (%s)p[(f0 + w + 4 * k) * %lldll] : 0; }\n",
                      type, type, l, (long long)L.sb, l, word, sf);
             stage += buf;
@@ -109,8 +109,8 @@ int jit_cwise_tile_source(const CwProgram& P, unsigned mask, bool wide, bool nt,
             direct += "    R v" + n + "[PER];\n";
             snprintf(buf, sizeof(buf),
                      "    { const %s* p = (const %s*)A.leaf[%d] + b * %lldll + (f0 + lane) * %lldll;\n#pragma unroll\n"
-                     "      for (int k = 0; k < PER; ++k) v%d[k] = (f0 + lane < F && s0 + w + 4 * k < S)"
-                     " ? (R)p[(s0 + w + 4 * k) * %lldll] : 0; }\n",
+                     "      for (int k = 0; k < PER; ++k) v%d[k] = (f0 + lane < F && ts0 + w + 4 * k < S)"
+                     " ? (R)p[(ts0 + w + 4 * k) * %lldll] : 0; }\n",
                      type, type, l, (long long)L.sb, sf, l, ss);
             loads += buf;
         }
@@ -153,17 +153,17 @@ int jit_cwise_tile_source(const CwProgram& P, unsigned mask, bool wide, bool nt,
            "    const long long m = A.by_xcd ? (h & 7) + 8 * ((h >> 3) / NT) : h / NT;\n"
            "    const long long tile = A.by_xcd ? (h >> 3) % NT : h % NT;\n"
            "    if (m >= NB) return;\n"
-           "    const long long b = m, ft = tile % NF, f0 = ft * TILE, s0 = tile / NF * TILE;\n" + scalars + direct + loads + stage +
+           "    const long long b = m, ft = tile % NF, f0 = ft * TILE, ts0 = tile / NF * TILE;\n" + scalars + direct + loads + stage +
            fill + "    __syncthreads();\n"
            "    " + dtype + "* const q = (" + dtype + "*)A.dst + b * (F * S) + (f0 + lane);\n"
            "    if (f0 + lane >= F) return;\n"
            "#pragma unroll\n"
            "    for (int k = 0; k < PER; ++k) {\n"
-           "        if (s0 + w + 4 * k >= S) break;\n"
-           "        R acc = 0, t = 0, s0_ = 0, s1 = 0, s2 = 0, s3 = 0;\n"
-           "        (void)t; (void)s0_; (void)s1; (void)s2; (void)s3;\n"
-           "#define s0 s0_\n" + prog + "#undef s0\n"
-           "        " + dtype + "* const p = q + (s0 + w + 4 * k) * F;\n"
+           "        if (ts0 + w + 4 * k >= S) break;\n"
+           "        R acc = 0, t = 0, s0 = 0, s1 = 0, s2 = 0, s3 = 0;\n"
+           "        (void)t; (void)s0; (void)s1; (void)s2; (void)s3;\n"
+           + prog +
+           "        " + dtype + "* const p = q + (ts0 + w + 4 * k) * F;\n"
            "        { " + store + " }\n"
            "    }\n"
            "}\n";
