@@ -151,6 +151,7 @@ def main():
     cg.solve(bd, xd, ctx=ctx)
     ctx.sync()
     cg.setMaxIterations(args.steps)
+    cm.reset_counters()
     ctx.sync()
     t0 = time.perf_counter()
     cg.solve(bd, xd, ctx=ctx)
@@ -161,10 +162,16 @@ def main():
     iters_per_s = args.steps / sec
     ms_per_step = 1000.0 * sec / args.steps
     # the reference's loop over CSR, fused: what "effective" counts (it can pass
-    # the HBM rate, since the solve reads the matrix by diagonals, without
-    # indices, from its 25th iteration on); and what that form moves
+    # the HBM rate where the solve reads the matrix by diagonals, without
+    # indices); and what the three launches move, iteration by iteration: the
+    # matrix as CSR or by diagonals, p and A p of the product, 16 + 24 bytes an
+    # unknown of the two updates (the two-launch form moves other bytes)
     cg_bytes = 8 * nnz + 56 * n
-    cg_dia_bytes = (5 * 4 + 8 + 16 + 24) * n
+    over_diagonals = cm.counters()["CgDiagonals"]
+    cg_moved = None
+    if args.cg_path == 1:
+        csr_iter, dia_iter = 8 * nnz + (4 + 8 + 16 + 24) * n, (5 * 4 + 8 + 16 + 24) * n
+        cg_moved = ((args.steps - over_diagonals) * csr_iter + over_diagonals * dia_iter) / sec / 1e9
     log(f"CG 2048^2: {iters_per_s:.1f} it/s, {ms_per_step * 1000:.1f} us/it, "
         f"{cg_bytes / (ms_per_step * 1e-3) / 1e9:.0f} GB/s (fused-minimum bytes)")
 
@@ -215,7 +222,8 @@ def main():
         "config": {"workload": "Jacobi-PCG iteration on 2D Poisson 2048x2048 (n=4194304, nnz=20963328), FP32 CSR",
                    "n": n, "nnz": nnz, "cg_bytes_per_iteration": cg_bytes,
                    "cg_effective_GBps": round(cg_bytes / (ms_per_step * 1e-3) / 1e9, 1),
-                   "cg_moved_GBps": round(cg_dia_bytes / (ms_per_step * 1e-3) / 1e9, 1),
+                   "cg_moved_GBps": None if cg_moved is None else round(cg_moved, 1),
+                   "cg_iterations_over_diagonals": over_diagonals,
                    "cg_128x128_tol1e-6": cfg1},
         "roofline": {"bound": "hbm", "kernel": "csr_spmv_kernel<float,float> (2048^2 Poisson)",
                      "achieved": round(spmv_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
