@@ -1187,8 +1187,12 @@ int cm_pcg_solve(cm_ctx_t ctx, int dtype, int n, int nnz, int batches, const int
     // launches; walking the CSR rows (matrices that are not banded) it equals
     // the launches at ~6000 rows. Up to 2^17 unknowns (n x batches) an
     // iteration is launch-bound and the two-launch form wins despite its
-    // tripled gathers (us per iteration, three / two launches: 128^2 12.6 /
-    // 10.2, 256^2 13.0 / 10.2, 512^2 13.8 / 13.7, 1024^2 26.9 / 33.1)
+    // tripled gathers (us per iteration over CSR, three / two launches: 128^2
+    // 12.6 / 10.2, 256^2 13.0 / 10.2, 512^2 13.8 / 13.7, 1024^2 26.9 / 33.1).
+    // The limit is that of matrices that stay on CSR: over the diagonals two
+    // launches also win above it (800 iterations: 128^2 12.4 / 8.4, 512^2 13.2 /
+    // 9.8, 1024^2 21.4 / 17.2, 512^2 with 8 right-hand sides 29.4 / 25.4), but which
+    // form a matrix will take is known only once its solve runs
     if (path == CM_CG_AUTO)
         path = (resident_ok && n <= 6144) ? CM_CG_RESIDENT
                                           : ((long long)n * batches <= (1 << 17) ? CM_CG_FUSED : CM_CG_MULTIKERNEL);

@@ -838,7 +838,7 @@ __global__ __launch_bounds__(CG_BS) void cg_iter_kernel(int n, int it, int B, in
 // the row bounds, the entries and the gathers in turn. Here everything but
 // the evaluation's partials has a known address, so the first rows' loads and
 // the state are requested together, before the state is looked at.
-// Measured on MI355X, us per launch at 128^2 FP32: 5.9 -> 3.8 (an empty launch
+// Measured on MI355X, us per launch at 128^2 FP32: 5.9 -> 3.5 (an empty launch
 // is 2 to 3 of them); whole iterations 9.9 -> 8.0 to 8.5, 360^2 10.8 -> 8.8, FP64 128^2
 // 11.3 -> 9.0, 8 right-hand sides of 128^2 13.1 -> 9.5. One element per thread in
 // KB (four times the blocks) changed nothing. The two-launch form has one matrix

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(SPMV_BS, sizeof(T) == 4 ? 8 : 4) void csr_spmv_mult
 // Row by row, a row of 27 entries is one load per lane, 37 lanes idle, and a
 // wave reduction; the next row's loads wait for it. Measured on MI355X, us, row
 // by row / windows: 27 points, 572 k rows, FP64 136 / 45.5 (one vector), 332 /
-// 68.1 (three, the windows read once for all), FP32 107 / 34.1; 200 k rows of 1
+// 67.3 (three, the windows read once for all), FP32 107 / 34.1; 200 k rows of 1
 // to 39 entries FP32 41.5 / 19.3. Without the next window's loads in flight
 // 54.8, 78.8, 46.5 and 23.8.
 //
